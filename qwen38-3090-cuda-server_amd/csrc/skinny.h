@@ -151,8 +151,6 @@ __device__ __forceinline__ void best_fold(Best& bs, int jj, float v, int n) {
 // into key group p % 64 (one cache line per group); the last workgroup of a
 // group bumps the group counter, and the last group to finish folds the 64
 // groups, writes the indices and clears the state for the next call.
-// kRows: at least M.
-template <int kRows = 16>
 __device__ __forceinline__ void argmax_arrive(const SkinnyArgs& a, int p, Best& bs, int lane) {
   const int c = lane & 15, q = lane >> 4;
   const int grp = p % kKeyGroups;
@@ -185,33 +183,29 @@ __device__ __forceinline__ void argmax_arrive(const SkinnyArgs& a, int p, Best& 
     last = arrive_dev(gcnt) == in_grp - 1 && arrive_dev(done) == (uint32_t)(ngroups - 1);
   }
   if (!__builtin_amdgcn_readfirstlane((int)last)) return;
-  // The last workgroup folds the groups, lane g group g: a row's 64 keys in one
-  // load instruction, every row's load in flight at once. One lane reading them
-  // one after another cost 8 us a row (INT4 head of 248320 rows, M = 9: 207 -> 149 us).
-  static_assert(kKeyGroups == 64, "one lane per key group");
-  uint64_t key[kRows];
+  // The last workgroup folds the groups: lane 16 h + m takes row m of groups
+  // 16 h .. 16 h + 15, its loads in flight together, then the four quarters
+  // meet. One lane reading every key one after another cost 8 us a row (INT4
+  // head of 248320 rows, M = 9: 201 -> 129 us).
+  static_assert(kKeyGroups == 64, "16 groups per quarter of the wave");
+  uint64_t* const rkeys = a.keys + (size_t)q * 256 + c;   // row c, group 16 q
+  uint64_t key[16], best = 0;
 #pragma unroll
-  for (int m = 0; m < kRows; ++m) {
-    key[m] = 0;
-    if (m < a.M && lane < ngroups)
-      key[m] = __hip_atomic_load(&a.keys[lane * 16 + m], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int g2 = 0; g2 < 16; ++g2)   // zero for groups and rows that have none
+    key[g2] = __hip_atomic_load(&rkeys[16 * g2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int g2 = 0; g2 < 16; ++g2) {
+    best = key[g2] > best ? key[g2] : best;
+    __hip_atomic_store(&rkeys[16 * g2], (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 #pragma unroll
-  for (int m = 0; m < kRows; ++m) {
-    uint64_t best = key[m];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const uint64_t o = (uint64_t)__shfl_xor((unsigned long long)best, off, 64);
-      best = o > best ? o : best;
-    }
-    if (lane == 0 && m < a.M) static_cast<int32_t*>(a.y)[m] = (int32_t)(~(uint32_t)(best & 0xffffffffu));
+  for (int off = 16; off < 64; off <<= 1) {
+    const uint64_t o = (uint64_t)__shfl_xor((unsigned long long)best, off, 64);
+    best = o > best ? o : best;
   }
-  if (lane < ngroups) {
-    for (int m = 0; m < a.M; ++m)
-      __hip_atomic_store(&a.keys[lane * 16 + m], (uint64_t)0, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    clear_dev(a.counters + (size_t)lane * kCounterStride);
-  }
+  if (lane < 16 && lane < a.M)
+    static_cast<int32_t*>(a.y)[lane] = (int32_t)(~(uint32_t)(best & 0xffffffffu));
+  if (lane < ngroups) clear_dev(a.counters + (size_t)lane * kCounterStride);
   if (lane == 0) clear_dev(a.counters + (size_t)kKeyGroups * kCounterStride);
 }
 

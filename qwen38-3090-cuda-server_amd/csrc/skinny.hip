@@ -919,7 +919,7 @@ __global__ __launch_bounds__(64 * W) void k_dec(SkinnyArgs a) {
     ++cu;
   }
   wait_vm<0>();   // no load lands in LDS after the workgroup released it
-  if (OUT == OUT_ARGMAX && wave == 0) argmax_arrive<1>(a, p, bs, lane);
+  if (OUT == OUT_ARGMAX && wave == 0) argmax_arrive(a, p, bs, lane);
 }
 
 // ------------------------------------------------------------- host side
