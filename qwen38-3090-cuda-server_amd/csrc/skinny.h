@@ -518,7 +518,7 @@ void allow_lds(int bytes) {
 
 // k_rows_xr (rows_xr.hip): launches it for these arguments (P and U filled in)
 // and returns true, or returns false where it does not apply.
-bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, int tS, int tD, hipStream_t st);
+bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, hipStream_t st);
 void rows_xr_prepare();   // raises its kernels' dynamic LDS limits on this device
 
 }  // namespace qw4

@@ -1318,6 +1318,7 @@ void prepare_dma_lds() {
     prepare_dec<OUT_RES>();
     prepare_dec<OUT_SWIGLU>();
     prepare_dec<OUT_NORM>();
+    rows_xr_prepare();
     prepare_gm<OUT_BF16>();
     prepare_gm<OUT_F32>();
     prepare_gm<OUT_RES>();
@@ -1460,6 +1461,11 @@ int run_skinny(void* y, const WeightView& w, const uint16_t* x, int M, qw4_scrat
       QW4_LAUNCH_CHECK();
       return QW4_OK;
     }
+  }
+  // activations in registers where that is the faster form (policy only)
+  if (mode == 0 && rows_xr_launch(OUT, FMT, a, device_cus(), (hipStream_t)stream)) {
+    QW4_LAUNCH_CHECK();
+    return QW4_OK;
   }
   const Launch l = launch_for<OUT, FMT>(w.out_f, w.G, M);
   // x must fit the LDS staging; beyond it, the caller's tmp path or an error
