@@ -18,36 +18,50 @@ namespace {
 
 constexpr int kEwThreads = 256;
 
-__global__ __launch_bounds__(kEwThreads) void k_rmsnorm(uint16_t* __restrict__ out,
-                                                        const uint16_t* __restrict__ x,
-                                                        const uint16_t* __restrict__ w,
-                                                        int dim, float eps) {
-  // thread t stands for the virtual threads t + 256 k of the shared order
-  // (norm_sumsq): virtual wave wave + 4 k
-  constexpr int kPer = kNormVThreads / kEwThreads;
-  const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// One workgroup of T threads per row. Thread t stands for the virtual threads
+// t + T k of the shared order (norm_sumsq), virtual wave wave + (T / 64) k. Their
+// first chunks of x and w (all of a row up to 8192) are loaded together and
+// kept for the output, so a row costs one memory latency. Rows of 5120, us: 1 row
+// 3.5 -> 2.3, 200 4.5 -> 3.0 (T = 1024); 1000 7.7 -> 7.1, 4096 21.5 -> 17.9 (T = 256;
+// 1024 threads take 7.7 and 21.6 there).
+template <int T>
+__global__ __launch_bounds__(T) void k_rmsnorm(uint16_t* __restrict__ out,
+                                               const uint16_t* __restrict__ x,
+                                               const uint16_t* __restrict__ w, int dim, float eps) {
+  constexpr int kPer = kNormVThreads / T;
+  const int row = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int kc = dim / 8;
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + (size_t)row * dim);
+  const u32x4* wr = reinterpret_cast<const u32x4*>(w);
+  u32x4* orow = reinterpret_cast<u32x4*>(out + (size_t)row * dim);
   __shared__ float vsum[kNormVWaves];
+  u32x4 xv[kPer], wv[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    float ss = 0.f;
-    for (int i = threadIdx.x + kEwThreads * k; i < kc; i += kNormVThreads) ss = norm_sumsq(ss, xr[i]);
+    const int i = min(t + T * k, kc - 1);
+    xv[k] = xr[i];
+    wv[k] = wr[i];
+  }
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    float ss = t + T * k < kc ? norm_sumsq(0.f, xv[k]) : 0.f;
+    for (int i = t + T * k + kNormVThreads; i < kc; i += kNormVThreads) ss = norm_sumsq(ss, xr[i]);
     ss = norm_wave_sum(ss);
-    if (lane == 0) vsum[wave + (kEwThreads / 64) * k] = ss;
+    if (lane == 0) vsum[wave + (T / 64) * k] = ss;
   }
   __syncthreads();
   const float inv = norm_inv(vsum, dim, eps);
-  const u32x4* wr = reinterpret_cast<const u32x4*>(w);
-  u32x4* orow = reinterpret_cast<u32x4*>(out + (size_t)row * dim);
-  for (int i = threadIdx.x; i < kc; i += kEwThreads) {
-    const u32x4 v = xr[i], g = wr[i];
+  auto store = [&](int i, const u32x4& v, const u32x4& g) {
     u32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       o[e] = pack_bf16x2(rmsnorm_f32(v[e], g[e], inv), rmsnorm_f32(v[e] >> 16, g[e] >> 16, inv));
     orow[i] = o;
-  }
+  };
+#pragma unroll
+  for (int k = 0; k < kPer; ++k)
+    if (t + T * k < kc) store(t + T * k, xv[k], wv[k]);
+  for (int i = t + kNormVThreads; i < kc; i += T) store(i, xr[i], wr[i]);
 }
 
 // out[i] = bf16(out[i] + x[i])
@@ -104,7 +118,12 @@ int qw4_rmsnorm(uint16_t* out, const uint16_t* x, const uint16_t* w, int rows, i
   if (rows < 0 || dim <= 0 || dim % 8) return QW4_ERR_SHAPE;
   if (((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) & 15) return QW4_ERR_ALIGN;
   if (rows == 0) return QW4_OK;
-  k_rmsnorm<<<rows, kEwThreads, 0, (hipStream_t)stream>>>(out, x, w, dim, eps);
+  // few rows: one virtual thread per thread, for latency; from about two
+  // workgroups of 1024 per CU on, smaller workgroups balance better
+  if (rows <= 512)
+    k_rmsnorm<kNormVThreads><<<rows, kNormVThreads, 0, (hipStream_t)stream>>>(out, x, w, dim, eps);
+  else
+    k_rmsnorm<kEwThreads><<<rows, kEwThreads, 0, (hipStream_t)stream>>>(out, x, w, dim, eps);
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }
