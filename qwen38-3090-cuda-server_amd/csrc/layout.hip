@@ -23,94 +23,143 @@ namespace {
 __device__ __forceinline__ int awq_slot(int e) { return slot_of_elem(e); }
 
 // ------------------------------------------------------------------ repack
-// One thread per destination word. Source layouts:
+// Source layouts:
 //   0 = compressed-tensors [N][K/8] (element e at slot e; w4a16_unpack.h:25-29)
 //   1 = AWQ packed along K [K/8][N], 2 = AWQ packed along N [K][N/8].
-template <int SRC>
-__global__ void k_repack_q(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
-                           int n_src, int K, int G, int tile0) {
-  const size_t per_tile = (size_t)G * kWordsPerBlock;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)(n_src / kTileN) * per_tile) return;
-  const int bl = (int)(t / per_tile);
-  const int rem = (int)(t % per_tile);
-  const int g = rem >> 10, j = (rem >> 8) & 3, p = (rem >> 2) & 63, w = rem & 3;
-  const int ns = bl * kTileN + tile_row_of_pos(p);     // source row
-  const int r = g * 16 + 4 * j + w;                    // word of the row: k = 8r..8r+7
-  uint32_t out = 0;
-  if (SRC == 0) {
-    const uint32_t s = src[(size_t)ns * (K / 8) + r];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out |= ((s >> (4 * e)) & 0xFu) << (4 * slot_of_elem(e));
-  } else if (SRC == 1) {
-    const uint32_t s = src[(size_t)r * n_src + ns];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out |= ((s >> (4 * awq_slot(e))) & 0xFu) << (4 * slot_of_elem(e));
-  } else {
-    const int sh = 4 * awq_slot(ns & 7);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t s = src[(size_t)(8 * r + e) * (n_src / 8) + (ns >> 3)];
-      out |= ((s >> sh) & 0xFu) << (4 * slot_of_elem(e));
-    }
-  }
-  dst[(size_t)(tile0 + bl) * per_tile + rem] = out;
+// Nibbles of a compressed-tensors word (element e at nibble e) in slot order:
+// the even elements in the low half, the odd ones in the high half.
+__device__ __forceinline__ uint32_t ct_to_slots(uint32_t s) {
+  uint32_t ev = s & 0x0F0F0F0Fu, od = (s >> 4) & 0x0F0F0F0Fu;
+  ev = (ev | (ev >> 4)) & 0x00FF00FFu;
+  od = (od | (od >> 4)) & 0x00FF00FFu;
+  return ((ev | (ev >> 8)) & 0xFFFFu) | ((od | (od >> 8)) << 16);
 }
 
-// One thread per (tile, group, 4-row quad): scales and zero points.
+// One wave per (tile, kRepackGroups groups), lane p at storage position p (row
+// 4 (p % 16) + p / 16): whole 1 KiB of a block per store, and for source 0 the
+// 128 contiguous bytes of a row that one lane needs. The scale records and
+// zero points of the same groups go with them (lane r at row r), so a repack
+// is one launch. Bound by memory: 5120x5120 compressed-tensors, 27 MB
+// moved, 23 us in two launches with one thread per word, 10.2 us so.
+constexpr int kRepackGroups = 2;
+
 template <int SRC>
-__global__ void k_repack_meta(uint16_t* __restrict__ dscale, uint16_t* __restrict__ dzero,
-                              const uint16_t* __restrict__ sscale,
-                              const uint32_t* __restrict__ szero, int n_src, int G,
-                              int tile0) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (n_src / kTileN) * G * 16) return;
-  const int bl = t / (G * 16), g = (t / 16) % G, c = t & 15;
-  const size_t blk = (size_t)(tile0 + bl) * G + g;
-  uint32_t z = 0;
+__global__ __launch_bounds__(256) void k_repack(uint32_t* __restrict__ dst,
+                                                uint16_t* __restrict__ dscale,
+                                                uint16_t* __restrict__ dzero,
+                                                const uint32_t* __restrict__ src,
+                                                const uint16_t* __restrict__ sscale,
+                                                const uint32_t* __restrict__ szero, int n_src,
+                                                int K, int G, int tile0) {
+  const int lane = threadIdx.x & 63;
+  const int per_tile = (G + kRepackGroups - 1) / kRepackGroups;
+  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (item >= (n_src / kTileN) * per_tile) return;
+  const int bl = item / per_tile, g0 = (item % per_tile) * kRepackGroups;
+  const int ns = bl * kTileN + tile_row_of_pos(lane);   // source row of position `lane`
+  u32x4 q[kRepackGroups][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int ns = bl * kTileN + 4 * c + i;
-    uint16_t s;
-    uint32_t zn;
-    if (SRC == 0) {
-      s = sscale[(size_t)ns * G + g];
-      zn = (szero[(size_t)(ns >> 3) * G + g] >> (4 * (ns & 7))) & 0xFu;  // w4a16_unpack.h:38-42
-    } else {
-      s = sscale[(size_t)g * n_src + ns];
-      zn = (szero[(size_t)g * (n_src / 8) + (ns >> 3)] >> (4 * awq_slot(ns & 7))) & 0xFu;
+  for (int i = 0; i < kRepackGroups; ++i) {
+    const int g = min(g0 + i, G - 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = g * 16 + 4 * j;   // words r .. r + 3 of the row: k = 8 r .. 8 r + 31
+      if (SRC == 0) {
+        const uint32_t* s = src + (size_t)ns * (K / 8) + r;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) q[i][j][w] = s[w];
+      } else if (SRC == 1) {   // the AWQ slot order is the repacked one
+#pragma unroll
+        for (int w = 0; w < 4; ++w) q[i][j][w] = src[(size_t)(r + w) * n_src + ns];
+      } else {
+        const int sh = 4 * awq_slot(ns & 7);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          uint32_t o = 0;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t s = src[(size_t)(8 * (r + w) + e) * (n_src / 8) + (ns >> 3)];
+            o |= ((s >> sh) & 0xFu) << (4 * slot_of_elem(e));
+          }
+          q[i][j][w] = o;
+        }
+      }
     }
-    dscale[blk * kMetaU16 + 4 * c + i] = s;
-    z |= zn << (4 * i);
   }
-  dzero[blk * 16 + c] = (uint16_t)z;
-  dscale[blk * kMetaU16 + 64 + c] = (uint16_t)z;
+#pragma unroll
+  for (int i = 0; i < kRepackGroups; ++i) {
+    const int g = g0 + i;
+    if (g >= G) break;
+    const size_t blk = (size_t)(tile0 + bl) * G + g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      u32x4 o = q[i][j];
+      if (SRC == 0)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) o[w] = ct_to_slots(o[w]);
+      *reinterpret_cast<u32x4*>(dst + blk * kWordsPerBlock + j * 256 + lane * 4) = o;
+    }
+    const int rn = bl * kTileN + lane;   // source row of the record's lane
+    uint16_t sc;
+    uint32_t z;
+    if (SRC == 0) {
+      sc = sscale[(size_t)rn * G + g];
+      z = (szero[(size_t)(rn >> 3) * G + g] >> (4 * (rn & 7))) & 0xFu;  // w4a16_unpack.h:38-42
+    } else {
+      sc = sscale[(size_t)g * n_src + rn];
+      z = (szero[(size_t)g * (n_src / 8) + (rn >> 3)] >> (4 * awq_slot(rn & 7))) & 0xFu;
+    }
+    dscale[blk * kMetaU16 + lane] = sc;
+    // four rows' zero points to a u16
+    z <<= 4 * (lane & 3);
+    z |= __shfl_xor(z, 1, 64);
+    z |= __shfl_xor(z, 2, 64);
+    if ((lane & 3) == 0) {
+      dzero[blk * 16 + (lane >> 2)] = (uint16_t)z;
+      dscale[blk * kMetaU16 + 64 + (lane >> 2)] = (uint16_t)z;
+    }
+  }
 }
 
 // ----------------------------------------------------------------- dequant
-// dst [nrows][K] = RNE(float(q - z) * s), one thread per 8 consecutive k.
-__global__ void k_dequant_rows(uint16_t* __restrict__ dst, const uint32_t* __restrict__ qw,
-                               const uint16_t* __restrict__ sc,
-                               const uint16_t* __restrict__ zr, int row0, int nrows,
-                               int K, int G) {
-  const int wpr = K / 8;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)nrows * wpr) return;
-  const int r = (int)(t / wpr), wi = (int)(t % wpr);
-  const int n = row0 + r, b = n >> 6, rr = n & 63;
-  const int g = wi >> 4, j = (wi >> 2) & 3, w = wi & 3;
+// dst [nrows][K] = RNE(float(q - z) * s). One workgroup per (tile, kDeqGroups
+// groups), so a block's lines are read by one CU and every 16 lanes write 256
+// bytes of a row; one thread per 8 consecutive k. Bound by the bf16 store:
+// 7168x5120, 73 MB: 23 us with one thread per word along a row, 16.6 us so.
+constexpr int kDeqGroups = 2;
+
+__global__ __launch_bounds__(256) void k_dequant_rows(uint16_t* __restrict__ dst,
+                                                      const uint32_t* __restrict__ qw,
+                                                      const uint16_t* __restrict__ sc,
+                                                      const uint16_t* __restrict__ zr, int row0,
+                                                      int nrows, int K, int G) {
+  const int per_tile = (G + kDeqGroups - 1) / kDeqGroups;
+  const int b = (row0 >> 6) + (int)blockIdx.x / per_tile;   // tile
+  const int g0 = ((int)blockIdx.x % per_tile) * kDeqGroups;
+  // thread: word wi of its group (of kDeqGroups), row `rs` of every 256 / (16
+  // kDeqGroups) rows
+  constexpr int kRows = 256 / (16 * kDeqGroups);
+  const int wi = threadIdx.x % (16 * kDeqGroups), rs = threadIdx.x / (16 * kDeqGroups);
+  const int g = g0 + wi / 16, j = (wi >> 2) & 3, w = wi & 3;
+  if (g >= G) return;
   const size_t blk = (size_t)b * G + g;
-  const uint32_t word = qw[blk * kWordsPerBlock + j * 256 + tile_pos_of_row(rr) * 4 + w];
-  const float s = bf16_bits_to_f32(sc[blk * kMetaU16 + rr]);
-  const int z = (zr[blk * 16 + (rr >> 2)] >> (4 * (rr & 3))) & 0xF;
-  uint32_t o[4];
 #pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const float a = (float)((int)((word >> (4 * slot_of_elem(e))) & 0xFu) - z) * s;
-    const float c = (float)((int)((word >> (4 * slot_of_elem(e + 1))) & 0xFu) - z) * s;
-    o[e / 2] = pack_bf16x2(a, c);
+  for (int it = 0; it < kTileN / kRows; ++it) {
+    const int rr = rs + kRows * it, n = b * kTileN + rr;   // row of the tile, of the tensor
+    if (n < row0 || n >= row0 + nrows) continue;
+    const uint32_t word = qw[blk * kWordsPerBlock + j * 256 + tile_pos_of_row(rr) * 4 + w];
+    const float s = bf16_bits_to_f32(sc[blk * kMetaU16 + rr]);
+    const int z = (zr[blk * 16 + (rr >> 2)] >> (4 * (rr & 3))) & 0xF;
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const float a = (float)((int)((word >> (4 * slot_of_elem(e))) & 0xFu) - z) * s;
+      const float c = (float)((int)((word >> (4 * slot_of_elem(e + 1))) & 0xFu) - z) * s;
+      o[e / 2] = pack_bf16x2(a, c);
+    }
+    *reinterpret_cast<u32x4*>(dst + (size_t)(n - row0) * K + (size_t)g * kGroup + 8 * (4 * j + w)) =
+        u32x4{o[0], o[1], o[2], o[3]};
   }
-  *reinterpret_cast<u32x4*>(dst + (size_t)r * K + 8 * wi) = u32x4{o[0], o[1], o[2], o[3]};
 }
 
 // ------------------------------------------------------- INT4 quantizer
@@ -463,20 +512,17 @@ static int repack_into(qw4_weights* w, int row_offset, const uint32_t* q, const 
     return QW4_ERR_SHAPE;
   hipStream_t hs = (hipStream_t)stream;
   const int G = w->num_groups, tile0 = row_offset / kTileN;
-  const size_t nq = (size_t)(out_f / kTileN) * G * kWordsPerBlock;
-  const size_t nm = (size_t)(out_f / kTileN) * G * 16;
+  const size_t items = (size_t)(out_f / kTileN) * ((G + kRepackGroups - 1) / kRepackGroups);
+  const unsigned nb = blocks_for(items, 4);
   switch (src) {
     case 0:
-      k_repack_q<0><<<blocks_for(nq, 256), 256, 0, hs>>>(w->qweight, q, out_f, w->in_f, G, tile0);
-      k_repack_meta<0><<<blocks_for(nm, 256), 256, 0, hs>>>(w->scale, w->zeros, s, z, out_f, G, tile0);
+      k_repack<0><<<nb, 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
       break;
     case QW4_LAYOUT_AWQ_K:
-      k_repack_q<1><<<blocks_for(nq, 256), 256, 0, hs>>>(w->qweight, q, out_f, w->in_f, G, tile0);
-      k_repack_meta<1><<<blocks_for(nm, 256), 256, 0, hs>>>(w->scale, w->zeros, s, z, out_f, G, tile0);
+      k_repack<1><<<nb, 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
       break;
     case QW4_LAYOUT_AWQ_N:
-      k_repack_q<2><<<blocks_for(nq, 256), 256, 0, hs>>>(w->qweight, q, out_f, w->in_f, G, tile0);
-      k_repack_meta<1><<<blocks_for(nm, 256), 256, 0, hs>>>(w->scale, w->zeros, s, z, out_f, G, tile0);
+      k_repack<2><<<nb, 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
       break;
     default:
       return QW4_ERR_LAYOUT;
@@ -511,9 +557,10 @@ int qw4_dequant_rows(uint16_t* dst, const qw4_weights* w, int row0, int nrows, v
   if (row0 < 0 || nrows < 0 || row0 + nrows > w->out_f) return QW4_ERR_SHAPE;
   if (((uintptr_t)dst & 15) != 0) return QW4_ERR_ALIGN;
   if (nrows == 0) return QW4_OK;
-  const size_t n = (size_t)nrows * (w->in_f / 8);
-  k_dequant_rows<<<blocks_for(n, 256), 256, 0, (hipStream_t)stream>>>(
-      dst, w->qweight, w->scale, w->zeros, row0, nrows, w->in_f, w->num_groups);
+  const int tiles = ((row0 + nrows - 1) >> 6) - (row0 >> 6) + 1;
+  const unsigned nb = (unsigned)tiles * ((w->num_groups + kDeqGroups - 1) / kDeqGroups);
+  k_dequant_rows<<<nb, 256, 0, (hipStream_t)stream>>>(dst, w->qweight, w->scale, w->zeros, row0, nrows,
+                                                      w->in_f, w->num_groups);
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }
