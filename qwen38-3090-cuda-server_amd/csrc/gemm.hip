@@ -27,9 +27,10 @@ int check_weights_public(const qw4_weights* w);
 namespace {
 
 // ---------------------------------------------------------------------------
-// k_gemm: 256 (M) x 256 (N) workgroup tile, v_mfma_f32_32x32x16_bf16 (the
+// k_gemm: 256 (M) x 256 (N) workgroup tile -- 32 MB (M) for MB = 2..7 m-blocks
+// where the rows do not fill 256 (gemm_plan) -- v_mfma_f32_32x32x16_bf16 (the
 // full-rate bf16 shape on gfx950). The default: 4 waves, one per SIMD, each a
-// whole 64-row weight tile against all 256 activation rows (its 256
+// whole 64-row weight tile against all the tile's activation rows (its 32 MB
 // accumulator registers in AGPRs); G2Split below lists the 8-wave forms.
 //
 //  * Weights are the MFMA A operand (rows = output columns n). Each wave loads
@@ -51,8 +52,7 @@ namespace {
 //    p = 16 (r % 4) + 8 b + 2 (r / 8) + (r / 4) % 2, so the four D rows a lane
 //    holds for each r / 8 are four consecutive output columns (an 8-byte
 //    piece of a staged row, see g2_store_staged).
-constexpr int G2_BM = 256, G2_BN = 256;
-constexpr int G2_ROWBLOCKS = G2_BM / 4;  // 1 KiB (4-row) activation loads per group
+constexpr int G2_BM = 256, G2_BN = 256;   // rows at most (32 MB of them, see G2Split), columns
 
 typedef float f32x16v __attribute__((ext_vector_type(16)));
 
@@ -78,19 +78,22 @@ struct GemmArgs {
 //  * NH = 2, NW = 4: one wave per SIMD owns a whole tile against all 8
 //    m-blocks (half the LDS reads, every weight dequantized once; its 256
 //    accumulator registers take the AGPR half of the register file).
-template <int NH, int NW>
+// MB: 32-row m-blocks of the workgroup's tile, 8 unless fewer rows need it.
+template <int NH, int NW, int MB>
 struct G2Split {
-  static constexpr int MBW = 64 / (NW * NH);         // m-blocks per wave
+  static constexpr int MBW = 8 * MB / (NW * NH);     // m-blocks per wave
   static constexpr int UNITS = NH * MBW;             // (half, m-block) pairs per wave
-  static constexpr int ACT = G2_ROWBLOCKS / NW;      // activation loads per wave and group
-  static constexpr int FIXP = 32 / NW;               // fixup blocks per wave region
+  static constexpr int ACT = 8 * MB / NW;            // 1 KiB (4-row) activation loads per wave and group
+  static constexpr int FIXP = (UNITS + 1) / 2;       // fixup blocks per wave region
+  // groups buffered: as many 8 MB KiB activation buffers as LDS holds, 4 at most
+  static constexpr int DEPTH = MB <= 4 ? 4 : MB == 5 ? 3 : 2;
   // k-step schedule (measured on MI355X at the config-4 shapes): VALU slots
   // after each MFMA, LDS operand reads after each of the first MFMAs, and the
   // k-steps that carry the next group's activation loads.
   static constexpr int VALU = NW == 8 ? 4 * NH : 2;
   static constexpr int DS = 2;
   static constexpr int ACTSTEPS = NW == 8 ? 4 : 8;
-  static_assert(MBW * NH * NW == 64 && ACT % 4 == 0, "unsupported split");
+  static_assert(MBW * NH * NW == 8 * MB && ACT * NW == 8 * MB, "unsupported split");
   __device__ static void coords(int wave, int& wt, int& b0, int& mw) {
     wt = NH == 1 ? (wave >> 1) : (wave & 3);   // tile of the 4 this wave owns
     b0 = NH == 1 ? (wave & 1) : 0;             // first tile half
@@ -139,24 +142,19 @@ __device__ __forceinline__ void g2_load_weights(WeightGroup<NH>& wg, const G2Rsr
   }
 }
 
-// Issue load i (of G2_ROWBLOCKS / NW) of this wave's share of the activation
-// rows of group g into buf. `act` covers rows [m0, M); rows past M lie outside
-// it and read as zeros. voff[i % 4] is the lane's byte offset of load i
-// relative to its first row (the swizzle repeats every 4 loads).
+// Issue activation load i of this wave (4 rows, 1 KiB) of group g into buf: row
+// block i NW + wave. `act` covers rows [m0, M); rows past M lie outside it and
+// read as zeros. voff is the lane's byte offset relative to a block's first
+// row: the swizzle repeats every 4 blocks, so it is the same for all of a
+// wave's.
 template <int NW>
-__device__ __forceinline__ void g2_load_act1(__amdgpu_buffer_rsrc_t act, const uint32_t (&voff)[4],
+__device__ __forceinline__ void g2_load_act1(__amdgpu_buffer_rsrc_t act, uint32_t voff,
                                              uint32_t row_bytes, u32x4* buf, int g, int wave,
                                              int i) {
-  const int rb = wave * (G2_ROWBLOCKS / NW) + i;
+  const int rb = i * NW + wave;
   __builtin_amdgcn_raw_ptr_buffer_load_lds(act, buf + rb * 64, 16,
-                                           voff[i & 3] + (uint32_t)(4 * rb) * row_bytes,
+                                           voff + (uint32_t)(4 * rb) * row_bytes,
                                            (uint32_t)g * (kGroup * 2), 0, 0);
-}
-template <int NW>
-__device__ __forceinline__ void g2_load_act(__amdgpu_buffer_rsrc_t act, const uint32_t (&voff)[4],
-                                            uint32_t row_bytes, u32x4* buf, int g, int wave) {
-#pragma unroll
-  for (int i = 0; i < G2_ROWBLOCKS / NW; ++i) g2_load_act1<NW>(act, voff, row_bytes, buf, g, wave, i);
 }
 
 // One packed word -> 8 bf16 weights RNE((q - z) s), c = -z s, in the order
@@ -210,23 +208,101 @@ __device__ __forceinline__ int g2_xcd_order(int blk, int count) {
   return (blk & 7) * (count >> 3) + (blk >> 3);
 }
 
-// One wave's share of one (tile, group range) segment: acc = sum over groups
-// [g0, g1) of this wave's weight rows x the tile's activation rows.
-template <int NH, int NW>
-__device__ __forceinline__ void g2_segment(const GemmArgs& a, const G2Rsrc& rs,
-                                           u32x4 (*lds)[G2_BM * 16],
-                                           f32x16v (&acc)[NH][G2Split<NH, NW>::MBW], int m0,
-                                           int ltile, int b0, int mw, int g0, int g1, int wave,
-                                           int lane) {
-  using Sp = G2Split<NH, NW>;
+// One group of a segment: the MFMAs of group g (its activation rows in buf, its
+// weights in cur) while the loads of a later group gn go out, activations into
+// nbuf and weights into nxt (actn, rsn: zero-length resources where there is no
+// such group -- they fetch nothing and need no branch, which would split the
+// k-step schedule).
+template <int NH, int NW, int MB>
+__device__ __forceinline__ void g2_group(const GemmArgs& a, f32x16v (&acc)[NH][G2Split<NH, NW, MB>::MBW],
+                                         const WeightGroup<NH>& cur, WeightGroup<NH>& nxt,
+                                         const u32x4* buf, u32x4* nbuf,
+                                         __amdgpu_buffer_rsrc_t actn, const G2Rsrc& rsn,
+                                         uint32_t voff, uint32_t row_bytes, int ltile, int b0, int gn,
+                                         int wave, int lane) {
+  using Sp = G2Split<NH, NW, MB>;
   constexpr int MBW = Sp::MBW;
   const int r = lane & 31, h = lane >> 5;
   const int zsh = 4 * (r & 3);
+  // Group gn's activation rows spread evenly over the first Sp::ACTSTEPS
+  // k-steps below, so that what the workgroup writes into LDS per group does
+  // not arrive in one burst on top of the first steps' operand reads (8
+  // waves: steps 0-3, 4% faster than one burst and 1.5% than one load per
+  // step; 4 waves: all 8 steps, equal to steps 0-3); its weights in k-steps
+  // kWStep.. kWStep + NH (0.5-0.8% faster than all at the group's start, where
+  // they delay its first MFMA).
+  float sf[NH], cf[NH];
+#pragma unroll
+  for (int j = 0; j < NH; ++j) {
+    sf[j] = bf16_bits_to_f32(cur.s[j]);
+    cf[j] = -(float)((cur.z[j] >> zsh) & 0xFu) * sf[j];
+  }
+  // Software pipeline over the group's 8 k-steps: the activation operands
+  // and the dequantized weight operands of step u + 1 are produced while
+  // step u's MFMAs run.
+  u32x4 xo[2][MBW];
+  bf16x8 wd[2][NH];
+#pragma unroll
+  for (int mb = 0; mb < MBW; ++mb) xo[0][mb] = buf[mb * 512 + ((4 * h) ^ (r & 15))];
+#pragma unroll
+  for (int j = 0; j < NH; ++j) wd[0][j] = g2_deq(cur.q[j][0][0], sf[j], cf[j]);
+  // Fence: the prologue's reads must not fill the DS slots of the pattern below.
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int cu = u & 1, nu = cu ^ 1;
+    constexpr int kWStep = 4;
+    if (u >= kWStep && u <= kWStep + NH)
+      g2_load_weights(nxt, rsn, a.G, ltile, b0, gn, lane, u - kWStep);
+    if (u < Sp::ACTSTEPS) {
+#pragma unroll
+      for (int i = Sp::ACT * u / Sp::ACTSTEPS; i < Sp::ACT * (u + 1) / Sp::ACTSTEPS; ++i)
+        g2_load_act1<NW>(actn, voff, row_bytes, nbuf, gn, wave, i);
+    }
+    if (u + 1 < 8) {
+      const int s1 = (u + 1) >> 2, t1 = (u + 1) & 3;
+      const int slot = (8 * s1 + 4 * h + t1) ^ (r & 15);
+#pragma unroll
+      for (int mb = 0; mb < MBW; ++mb) xo[nu][mb] = buf[mb * 512 + slot];
+#pragma unroll
+      for (int j = 0; j < NH; ++j) wd[nu][j] = g2_deq(cur.q[j][s1][t1], sf[j], cf[j]);
+    }
+#pragma unroll
+    for (int mb = 0; mb < MBW; ++mb)
+#pragma unroll
+      for (int j = 0; j < NH; ++j)
+        acc[j][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            wd[cu][j], __builtin_bit_cast(bf16x8, xo[cu][mb]), acc[j][mb], 0, 0, 0);
+    if (u + 1 < 8) {
+#pragma unroll
+      for (int i = 0; i < MBW * NH; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        if (i < (MBW + Sp::DS - 1) / Sp::DS) __builtin_amdgcn_sched_group_barrier(0x100, Sp::DS, 0);  // DS read
+        __builtin_amdgcn_sched_group_barrier(0x002, Sp::VALU, 0);  // VALU
+      }
+    }
+    // NW = 4: one scheduling region per k-step, so that the next step's
+    // operand reads stay under this step's MFMAs instead of sinking to their
+    // first use (with one wave per SIMD nothing else hides their latency).
+    if (NW == 4) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// One wave's share of one (tile, group range) segment: acc = sum over groups
+// [g0, g1) of this wave's weight rows x the tile's activation rows.
+template <int NH, int NW, int MB>
+__device__ __forceinline__ void g2_segment(const GemmArgs& a, const G2Rsrc& rs,
+                                           u32x4 (*lds)[32 * MB * 16],
+                                           f32x16v (&acc)[NH][G2Split<NH, NW, MB>::MBW], int m0,
+                                           int ltile, int b0, int mw, int g0, int g1, int wave,
+                                           int lane) {
+  using Sp = G2Split<NH, NW, MB>;
+  constexpr int MBW = Sp::MBW, D = Sp::DEPTH;
+  const int r = lane & 31;
 #pragma unroll
   for (int j = 0; j < NH; ++j)
 #pragma unroll
     for (int mb = 0; mb < MBW; ++mb) acc[j][mb] = f32x16v{};
-  WeightGroup<NH> cur, nxt;
   // Activation rows [m0, M): the buffer's end turns rows past M into zeros.
   const uint32_t row_bytes = (uint32_t)a.K * 2u;
   const __amdgpu_buffer_rsrc_t act = __builtin_amdgcn_make_buffer_rsrc(
@@ -238,91 +314,55 @@ __device__ __forceinline__ void g2_segment(const GemmArgs& a, const G2Rsrc& rs,
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.qw), 0, 0, 0x00020000),
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.sc), 0, 0, 0x00020000),
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.zr), 0, 0, 0x00020000)};
-  uint32_t voff[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 4 * i + (lane >> 4);                 // row within the 16-row swizzle period
-    const int c = (lane & 15) ^ (row & 15);
-    voff[i] = (uint32_t)(lane >> 4) * row_bytes + (uint32_t)c * 16u;
-  }
+  const int srow = 4 * (wave & 3) + (lane >> 4);   // row within the 16-row swizzle period
+  const uint32_t voff = (uint32_t)(lane >> 4) * row_bytes + (uint32_t)((lane & 15) ^ srow) * 16u;
   __syncthreads();   // the previous segment's last LDS reads are done
-  g2_load_act<NW>(act, voff, row_bytes, lds[0], g0, wave);
-  g2_load_weights(cur, rs, a.G, ltile, b0, g0, lane);
-  for (int g = g0; g < g1; ++g) {
-    g2_wait_vm0();
-    __syncthreads();
-    const int sb = (g - g0) & 1;
-    const u32x4* buf = lds[sb] + (32 * mw + r) * 16;
-    // Group g + 1's activation rows spread evenly over the first Sp::ACTSTEPS
-    // k-steps below, so that the 64 KiB the workgroup writes into LDS per
-    // group do not arrive in one burst on top of the first steps' operand
-    // reads (8 waves: steps 0-3, 4% faster than one burst and 1.5% than one
-    // load per step; 4 waves: all 8 steps, equal to steps 0-3); its weights
-    // in k-steps kWStep.. kWStep + NH (0.5-0.8% faster than all at the
-    // group's start, where they delay its first MFMA).
-    // Past the segment's last group the loads go through zero-length
-    // resources: they fetch nothing (out-of-range buffer loads return zeros)
-    // and need no branch, which would split the k-step schedule below.
-    const bool more = g + 1 < g1;
-    const __amdgpu_buffer_rsrc_t actn = more ? act : act_none;
-    const G2Rsrc rsn = more ? rs : rs_none;
-    float sf[NH], cf[NH];
+  if constexpr (D == 2) {
+    WeightGroup<NH> cur, nxt;
 #pragma unroll
-    for (int j = 0; j < NH; ++j) {
-      sf[j] = bf16_bits_to_f32(cur.s[j]);
-      cf[j] = -(float)((cur.z[j] >> zsh) & 0xFu) * sf[j];
+    for (int i = 0; i < Sp::ACT; ++i) g2_load_act1<NW>(act, voff, row_bytes, lds[0], g0, wave, i);
+    g2_load_weights(cur, rs, a.G, ltile, b0, g0, lane);
+    for (int g = g0; g < g1; ++g) {
+      g2_wait_vm0();
+      __syncthreads();
+      const int sb = (g - g0) & 1;
+      const bool more = g + 1 < g1;
+      g2_group<NH, NW, MB>(a, acc, cur, nxt, lds[sb] + (32 * mw + r) * 16, lds[sb ^ 1],
+                           more ? act : act_none, more ? rs : rs_none, voff, row_bytes, ltile, b0,
+                           g + 1, wave, lane);
+      cur = nxt;
     }
-    // Software pipeline over the group's 8 k-steps: the activation operands
-    // and the dequantized weight operands of step u + 1 are produced while
-    // step u's MFMAs run.
-    u32x4 xo[2][MBW];
-    bf16x8 wd[2][NH];
+  } else {
+    // D buffers, the loads D - 1 groups ahead: a group of few m-blocks computes
+    // in less than a memory latency. Unrolled by D, so that every buffer --
+    // LDS and weight registers -- is named statically and no register is
+    // copied (a copy would wait for its load). Waits are counted: loads
+    // complete in order, and every group issues the same number.
+    constexpr int kLoads = Sp::ACT + 4 * NH;
+    WeightGroup<NH> wg[D];
 #pragma unroll
-    for (int mb = 0; mb < MBW; ++mb) xo[0][mb] = buf[mb * 512 + ((4 * h) ^ (r & 15))];
+    for (int d = 0; d < D - 1; ++d) {
+      const bool in = g0 + d < g1;
 #pragma unroll
-    for (int j = 0; j < NH; ++j) wd[0][j] = g2_deq(cur.q[j][0][0], sf[j], cf[j]);
-    // Fence: the prologue's reads must not fill the DS slots of the pattern below.
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int cu = u & 1, nu = cu ^ 1;
-      constexpr int kWStep = 4;
-      if (u >= kWStep && u <= kWStep + NH)
-        g2_load_weights(nxt, rsn, a.G, ltile, b0, g + 1, lane, u - kWStep);
-      if (u < Sp::ACTSTEPS) {
-#pragma unroll
-        for (int i = 0; i < Sp::ACT / Sp::ACTSTEPS; ++i)
-          g2_load_act1<NW>(actn, voff, row_bytes, lds[sb ^ 1], g + 1, wave,
-                           Sp::ACT / Sp::ACTSTEPS * u + i);
-      }
-      if (u + 1 < 8) {
-        const int s1 = (u + 1) >> 2, t1 = (u + 1) & 3;
-        const int slot = (8 * s1 + 4 * h + t1) ^ (r & 15);
-#pragma unroll
-        for (int mb = 0; mb < MBW; ++mb) xo[nu][mb] = buf[mb * 512 + slot];
-#pragma unroll
-        for (int j = 0; j < NH; ++j) wd[nu][j] = g2_deq(cur.q[j][s1][t1], sf[j], cf[j]);
-      }
-#pragma unroll
-      for (int mb = 0; mb < MBW; ++mb)
-#pragma unroll
-        for (int j = 0; j < NH; ++j)
-          acc[j][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              wd[cu][j], __builtin_bit_cast(bf16x8, xo[cu][mb]), acc[j][mb], 0, 0, 0);
-      if (u + 1 < 8) {
-#pragma unroll
-        for (int i = 0; i < MBW * NH; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-          if (i < MBW / Sp::DS) __builtin_amdgcn_sched_group_barrier(0x100, Sp::DS, 0);  // DS read
-          __builtin_amdgcn_sched_group_barrier(0x002, Sp::VALU, 0);  // VALU
-        }
-      }
-      // NW = 4: one scheduling region per k-step, so that the next step's
-      // operand reads stay under this step's MFMAs instead of sinking to their
-      // first use (with one wave per SIMD nothing else hides their latency).
-      if (NW == 4) __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < Sp::ACT; ++i)
+        g2_load_act1<NW>(in ? act : act_none, voff, row_bytes, lds[d], g0 + d, wave, i);
+      g2_load_weights(wg[d], in ? rs : rs_none, a.G, ltile, b0, g0 + d, lane);
     }
-    cur = nxt;
+    for (int gb = g0; gb < g1; gb += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int g = gb + d;
+        if (g >= g1) break;
+        // group g has landed (the D - 2 groups behind it may be in flight) for
+        // every wave, and every wave is done with group g - 1's buffer
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * kLoads) : "memory");
+        constexpr int kBack = D - 1;
+        const bool more = g + kBack < g1;
+        g2_group<NH, NW, MB>(a, acc, wg[d], wg[(d + kBack) % D], lds[d] + (32 * mw + r) * 16,
+                             lds[(d + kBack) % D], more ? act : act_none, more ? rs : rs_none, voff,
+                             row_bytes, ltile, b0, g + kBack, wave, lane);
+      }
+    }
   }
 }
 
@@ -337,12 +377,12 @@ __device__ __forceinline__ void g2_segment(const GemmArgs& a, const G2Rsrc& rs,
 // CPR)) -- after a wait and a barrier, so that all waves are done with the
 // segment's operand reads and their loads have landed -- and reads it back
 // row by row. Measured: gate M = 4096 0.617 -> 0.601 ms.
-template <int NH, int NW>
+template <int NH, int NW, int MB>
 __device__ __forceinline__ void g2_store_staged(const GemmArgs& a,
-                                                const f32x16v (&acc)[NH][G2Split<NH, NW>::MBW],
+                                                const f32x16v (&acc)[NH][G2Split<NH, NW, MB>::MBW],
                                                 u32x4* lds, int m0, int tile, int b0, int mw,
                                                 bool valid, int wave, int lane) {
-  constexpr int MBW = G2Split<NH, NW>::MBW;
+  constexpr int MBW = G2Split<NH, NW, MB>::MBW;
   constexpr int CPR = NH * 4;                      // 16-byte chunks per staged row
   constexpr int ROWS = MBW * 32;
   constexpr int RPI = 64 / CPR;                    // rows per read-back instruction
@@ -395,11 +435,11 @@ __device__ __forceinline__ uint32_t g2_slot_off(int vp, int which, int wave, int
   return (uint32_t)(vp * 2 + which) * kSlotBytes + (uint32_t)((wave * units + idx) * 4096 + lane * 16);
 }
 
-template <int NH, int NW>
+template <int NH, int NW, int MB>
 __device__ __forceinline__ void g2_slot_store(__amdgpu_buffer_rsrc_t rs,
-                                              const f32x16v (&acc)[NH][G2Split<NH, NW>::MBW],
+                                              const f32x16v (&acc)[NH][G2Split<NH, NW, MB>::MBW],
                                               int vp, int which, int wave, int lane) {
-  constexpr int MBW = G2Split<NH, NW>::MBW;
+  constexpr int MBW = G2Split<NH, NW, MB>::MBW;
 #pragma unroll
   for (int j = 0; j < NH; ++j)
 #pragma unroll
@@ -432,15 +472,15 @@ __device__ __forceinline__ int g2_owner_of(const GemmArgs& a, int u) {
 // order, so that the loads of a tile split many ways overlap instead of
 // paying one memory latency per piece. Tiles a single workgroup covered were
 // stored by the main kernel.
-constexpr int kFixBlocksPerTile = 32;
 constexpr int kFixAhead = 4;
 
-template <int NH, int NW>
+template <int NH, int NW, int MB>
 __global__ __launch_bounds__(64) void k_gemm_fixup(GemmArgs a) {
-  using Sp = G2Split<NH, NW>;
+  using Sp = G2Split<NH, NW, MB>;
   constexpr int MBW = Sp::MBW;
-  constexpr int kPer = Sp::UNITS / Sp::FIXP;   // (half, m-block) pairs per block
-  static_assert(NW * Sp::FIXP == kFixBlocksPerTile && kPer == 2, "fixup split");
+  constexpr int kPer = 2;   // (half, m-block) pairs per block
+  constexpr int kFixBlocksPerTile = NW * Sp::FIXP;
+  static_assert(Sp::UNITS % kPer == 0, "whole pairs per block");
   const int ts = blockIdx.x / kFixBlocksPerTile;   // split tile full + ts
   const int wave = (blockIdx.x / Sp::FIXP) % NW;
   const int part = blockIdx.x % Sp::FIXP;
@@ -490,7 +530,7 @@ __global__ __launch_bounds__(64) void k_gemm_fixup(GemmArgs a) {
     }
   }
   // pair index j * MBW + mb (g2_slot_store's order)
-  const int m0 = tm * G2_BM;
+  const int m0 = tm * 32 * MB;
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
     const int idx = part * kPer + e, j = idx / MBW, mb = idx % MBW;
@@ -506,11 +546,12 @@ __global__ __launch_bounds__(64) void k_gemm_fixup(GemmArgs a) {
   }
 }
 
-template <int NH, int NW>
+template <int NH, int NW, int MB>
 __global__ __launch_bounds__(64 * NW, 1) void k_gemm(GemmArgs a) {
-  using Sp = G2Split<NH, NW>;
+  using Sp = G2Split<NH, NW, MB>;
   constexpr int MBW = Sp::MBW;              // m-blocks per wave
-  __shared__ u32x4 lds[2][G2_BM * 16];      // 2 x 64 KiB: [row][16 swizzled chunks]
+  constexpr int BM = 32 * MB;               // rows of a tile
+  __shared__ u32x4 lds[Sp::DEPTH][BM * 16];   // [row][16 swizzled chunks]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform
   const int lane = threadIdx.x & 63;
   int wt, b0, mw;
@@ -549,8 +590,8 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm(GemmArgs a) {
     const int tile = tn * 4 + wt;
     const bool valid = tile * kTileN < a.N;
     const int ltile = valid ? tile : (a.N / kTileN - 1);
-    g2_segment<NH, NW>(a, wr, lds, acc, tm * G2_BM, ltile, b0, mw, 0, a.G, wave, lane);
-    g2_store_staged<NH, NW>(a, acc, &lds[0][0], tm * G2_BM, tile, b0, mw, valid, wave, lane);
+    g2_segment<NH, NW, MB>(a, wr, lds, acc, tm * BM, ltile, b0, mw, 0, a.G, wave, lane);
+    g2_store_staged<NH, NW, MB>(a, acc, &lds[0][0], tm * BM, tile, b0, mw, valid, wave, lane);
   }
   for (int u = u0; u < u1;) {
     const int ts = u / a.G, g0 = u - ts * a.G;
@@ -560,11 +601,11 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm(GemmArgs a) {
     const int tile = tn * 4 + wt;
     const bool valid = tile * kTileN < a.N;
     const int ltile = valid ? tile : (a.N / kTileN - 1);
-    g2_segment<NH, NW>(a, wr, lds, acc, tm * G2_BM, ltile, b0, mw, g0, g1, wave, lane);
+    g2_segment<NH, NW, MB>(a, wr, lds, acc, tm * BM, ltile, b0, mw, g0, g1, wave, lane);
     if (g0 == 0 && g1 == a.G) {
-      g2_store_staged<NH, NW>(a, acc, &lds[0][0], tm * G2_BM, tile, b0, mw, valid, wave, lane);
+      g2_store_staged<NH, NW, MB>(a, acc, &lds[0][0], tm * BM, tile, b0, mw, valid, wave, lane);
     } else {
-      g2_slot_store<NH, NW>(rs, acc, vp, u == u0 ? 0 : 1, wave, lane);
+      g2_slot_store<NH, NW, MB>(rs, acc, vp, u == u0 ? 0 : 1, wave, lane);
     }
     u = ts * a.G + g1;
   }
@@ -595,6 +636,73 @@ std::atomic<int> g_gemm_schedule{-1};
 // waves of whole tiles against 128 rows. All three sum every output in the
 // same order, so their results are bitwise equal.
 std::atomic<int> g_gemm_variant{0};
+
+template <int NH, int NW, int MB>
+void launch_gemm(const GemmArgs& a, int grid, int nt, hipStream_t s) {
+  k_gemm<NH, NW, MB><<<grid, 64 * NW, 0, s>>>(a);
+  if (a.full != nt)   // the split tiles
+    k_gemm_fixup<NH, NW, MB><<<(nt - a.full) * NW * G2Split<NH, NW, MB>::FIXP, 64, 0, s>>>(a);
+}
+
+// How a call is cut: tiles of 32 mb rows, schedule (0 per tile, 1 stream-K, 2
+// hybrid, 3 split-K in S slices) and its cost.
+struct GemmPlan {
+  int mb, tiles_n, tiles_m, pick, S;
+  double cost;
+};
+
+// Time of one (tile, group) step by its m-blocks, relative to 8. Measured over
+// whole rounds of tiles (65536x5120, 256 and 1000 rows; us per 40 groups): 2 60,
+// 3 74, 4 91, 5 101, 6 110, 7 125, 8 145; 2 and 3 are charged a little more
+// for the memory latency that they expose when tiles are split.
+double step_cost(int mb) { return mb < 4 ? 0.38 + 0.06 * mb : 0.22 + 0.0975 * mb; }
+
+GemmPlan gemm_plan(int M, int N, long long G, int mb, int cus, bool ws_ok, int schedule) {
+  GemmPlan p{mb, (N + G2_BN - 1) / G2_BN, (M + 32 * mb - 1) / (32 * mb), 0, 0, 0.};
+  const int nt = p.tiles_n * p.tiles_m, rem = nt % cus;
+  // Schedules, costed in group-steps per CU (one tile x 128 step; measured on
+  // MI355X at the config-4 shapes):
+  //  * per tile: one workgroup per tile, ceil(nt / CUs) G;
+  //  * stream-K: one workgroup per CU, all nt G (tile, group) units split
+  //    evenly, nt G / CUs + 16 (two fp32 partial tiles written per
+  //    workgroup) + 0.1 per piece of a cut tile (k_gemm_fixup's blocks read
+  //    a tile's pieces one after another);
+  //  * hybrid: whole tiles for the floor(nt / CUs) full rounds, then the
+  //    other nt % CUs tiles split over the CUs: the same work, one partial
+  //    per workgroup (+8), CUs / (nt % CUs) pieces per cut tile;
+  //  * split-K (at most CUs / 2 tiles): every tile cut into the same S
+  //    k-slices, S = CUs / nt (P = nt S workgroups, a multiple of 8, at
+  //    least 4 groups per slice): G / S + 8 + 0.1 S. Against stream-K it
+  //    writes one partial per workgroup instead of up to two, and the
+  //    workgroups of an XCD share A at the same k (down M = 1024: 0.159
+  //    against 0.170-0.180 ms; down M = 512 0.094 against 0.102-0.107).
+  // A split schedule runs when it beats per-tile by 5% (qw4_tune_gemm
+  // forces one, for tests and tuning): gate M = 512, 136 tiles, costs 37.6
+  // against 40 and measured 0.880 against 0.842 PFLOP/s.
+  const double t_dp = (double)((nt + cus - 1) / cus) * G;
+  const double work = (double)nt * G / cus;
+  const double t_sk = work + 16.0 + 0.1 * ((cus + nt - 1) / nt + 1);
+  const double t_hy = work + 8.0 + 0.1 * (rem ? (cus + rem - 1) / rem + 1 : 0);
+  ws_ok = ws_ok && rem != 0 && (long long)nt * G < (1LL << 31);
+  const bool sk_ok = ws_ok && (long long)nt * G >= 2LL * cus;
+  const bool hy_ok = ws_ok && nt > cus && (long long)rem * G >= (long long)cus;
+  int S = 2 * nt <= cus ? (int)std::min<long long>(cus / nt, G >= 8 ? G / 4 : G / 2) : 0;
+  while (S >= 2 && (nt * S) % 8) --S;
+  const bool kk_ok = ws_ok && S >= 2;
+  const double t_kk = (double)G / (S > 0 ? S : 1) + 8.0 + 0.1 * S;
+  p.cost = t_dp;
+  if (schedule == -1) {
+    double best = 0.95 * t_dp;
+    if (sk_ok && t_sk < best) { p.pick = 1; p.cost = best = t_sk; }
+    if (hy_ok && t_hy < best) { p.pick = 2; p.cost = best = t_hy; }
+    if (kk_ok && t_kk < best) { p.pick = 3; p.cost = t_kk; }
+  } else if ((schedule == 1 && sk_ok) || (schedule == 2 && hy_ok) || (schedule == 3 && kk_ok)) {
+    p.pick = schedule;
+  }
+  p.S = S;
+  p.cost *= step_cost(mb);
+  return p;
+}
 
 }  // namespace
 }  // namespace qw4
@@ -643,90 +751,60 @@ int qw4_gemm(uint16_t* C, const qw4_weights* w, const uint16_t* A, int M, qw4_wo
   if ((size_t)M * w->in_f * 2 >= (1ull << 32) || (size_t)w->out_f * w->in_f / 2 >= (1ull << 32))
     return QW4_ERR_SHAPE;
   {
-    const int tiles_n = (w->out_f + G2_BN - 1) / G2_BN;
-    const int tiles_m = (M + G2_BM - 1) / G2_BM;
-    const int nt = tiles_n * tiles_m;
-    GemmArgs a{w->qweight, w->scale, w->zeros, A, C, nullptr, M, w->out_f, w->in_f,
-                w->num_groups, tiles_n, tiles_m, nt % 8 == 0, nt, nt, 0};
-    int grid = nt;
-    // Three schedules, costed in group-steps per CU (one 256 x 256 x 128
-    // tile step; measured on MI355X at the config-4 shapes):
-    //  * per tile: one workgroup per tile, ceil(nt / CUs) G;
-    //  * stream-K: one workgroup per CU, all nt G (tile, group) units split
-    //    evenly, nt G / CUs + 16 (two fp32 partial tiles written per
-    //    workgroup) + 0.1 per piece of a cut tile (k_gemm_fixup's blocks read
-    //    a tile's pieces one after another);
-    //  * hybrid: whole tiles for the floor(nt / CUs) full rounds, then the
-    //    other nt % CUs tiles split over the CUs: the same work, one partial
-    //    per workgroup (+8), CUs / (nt % CUs) pieces per cut tile;
-    //  * split-K (at most CUs / 2 tiles): every tile cut into the same S
-    //    k-slices, S = CUs / nt (P = nt S workgroups, a multiple of 8, at
-    //    least 2 groups per slice): G / S + 8 + 0.1 S. Against stream-K it
-    //    writes one partial per workgroup instead of up to two, and the
-    //    workgroups of an XCD share A at the same k (down M = 1024: 0.159
-    //    against 0.170-0.180 ms; down M = 512 0.094 against 0.102-0.107).
-    // A split schedule runs when it beats per-tile by 5% (qw4_tune_gemm
-    // forces one, for tests and tuning): gate M = 512, 136 tiles, costs 37.6
-    // against 40 and measured 0.880 against 0.842 PFLOP/s.
-    const int sk_env = g_gemm_schedule.load(std::memory_order_relaxed);
+    const int schedule = g_gemm_schedule.load(std::memory_order_relaxed);
+    const int variant = g_gemm_variant.load(std::memory_order_relaxed);
     const int cus = device_cus();
-    const long long G = w->num_groups;
-    const int rem = nt % cus;
-    const double t_dp = (double)((nt + cus - 1) / cus) * G;
-    const double work = (double)nt * G / cus;
-    const double t_sk = work + 16.0 + 0.1 * ((cus + nt - 1) / nt + 1);
-    const double t_hy = work + 8.0 + 0.1 * (rem ? (cus + rem - 1) / rem + 1 : 0);
-    const bool ws_ok = ws && ws->buf && ws->bytes >= gemm_workspace_need(cus) && cus % 8 == 0 &&
-                       rem != 0 && (long long)nt * G < (1LL << 31);
-    const bool sk_ok = ws_ok && (long long)nt * G >= 2LL * cus;
-    const bool hy_ok = ws_ok && nt > cus && (long long)rem * G >= (long long)cus;
-    int S = 2 * nt <= cus ? (int)std::min<long long>(cus / nt, G / 2) : 0;
-    while (S >= 2 && (nt * S) % 8) --S;
-    const bool kk_ok = ws_ok && S >= 2;
-    const double t_kk = (double)G / (S > 0 ? S : 1) + 8.0 + 0.1 * S;
-    int pick = 0;   // 0 per tile, 1 stream-K, 2 hybrid, 3 split-K
-    if (sk_env == 1 && sk_ok) pick = 1;
-    else if (sk_env == 2 && hy_ok) pick = 2;
-    else if (sk_env == 3 && kk_ok) pick = 3;
-    else if (sk_env == -1) {
-      double best = 0.95 * t_dp;
-      if (sk_ok && t_sk < best) { pick = 1; best = t_sk; }
-      if (hy_ok && t_hy < best) { pick = 2; best = t_hy; }
-      if (kk_ok && t_kk < best) pick = 3;
-    }
-    if (pick == 3) {
+    const bool ws_ok = ws && ws->buf && ws->bytes >= gemm_workspace_need(cus) && cus % 8 == 0;
+    GemmPlan p = gemm_plan(M, w->out_f, w->num_groups, 8, cus, ws_ok, schedule);
+    // Tiles of fewer rows where that costs less: rows that do not fill 256-row
+    // tiles (us, 256-row tiles against the plan's: gate|up 34816x5120 at 64 / 128 /
+    // 300 rows 98 / 98 / 150 -> 55 / 70 / 126, down 5120x17408 53 / 55 / 87 -> 30 / 39 /
+    // 66, o 5120x4096 36 / 36 / 40 -> 19 / 23 / 31), and few tiles, cut in fewer
+    // slices (o at 256 rows 37 -> 28). By 3% at least, what the model resolves:
+    // down at 2000 rows costs 100.9 in 224-row tiles against 101.3 and is 3% slower.
+    if (schedule == -1 && variant == 0)
+      for (int mb = 7; mb >= 2; --mb) {
+        const GemmPlan q = gemm_plan(M, w->out_f, w->num_groups, mb, cus, ws_ok, schedule);
+        if (q.cost < 0.97 * p.cost) p = q;
+      }
+    const int nt = p.tiles_n * p.tiles_m, mb = p.mb;
+    GemmArgs a{w->qweight, w->scale, w->zeros, A, C, nullptr, M, w->out_f, w->in_f,
+                w->num_groups, p.tiles_n, p.tiles_m, nt % 8 == 0, nt, nt, 0};
+    int grid = nt;
+    if (p.pick == 3) {
       a.slots = static_cast<float*>(ws->buf);
-      a.P = nt * S;
+      a.P = nt * p.S;
       a.full = 0;
-      a.U = (int)(nt * G);
+      a.U = nt * w->num_groups;
       a.map = 2;
       grid = a.P;
-    } else if (pick) {
+    } else if (p.pick) {
       a.slots = static_cast<float*>(ws->buf);
       a.P = cus;
-      a.full = pick == 2 ? nt - rem : 0;
-      a.U = (int)((nt - a.full) * G);
+      a.full = p.pick == 2 ? nt - nt % cus : 0;
+      a.U = (nt - a.full) * w->num_groups;
       a.map = 1;
       grid = cus;
     }
     hipStream_t s = (hipStream_t)stream;
-    const int variant = g_gemm_variant.load(std::memory_order_relaxed);
     if (variant == 1)
-      k_gemm<1, 8><<<grid, 512, 0, s>>>(a);
+      launch_gemm<1, 8, 8>(a, grid, nt, s);
     else if (variant == 2)
-      k_gemm<2, 8><<<grid, 512, 0, s>>>(a);
+      launch_gemm<2, 8, 8>(a, grid, nt, s);
+    else if (mb == 2)
+      launch_gemm<2, 4, 2>(a, grid, nt, s);
+    else if (mb == 3)
+      launch_gemm<2, 4, 3>(a, grid, nt, s);
+    else if (mb == 4)
+      launch_gemm<2, 4, 4>(a, grid, nt, s);
+    else if (mb == 5)
+      launch_gemm<2, 4, 5>(a, grid, nt, s);
+    else if (mb == 6)
+      launch_gemm<2, 4, 6>(a, grid, nt, s);
+    else if (mb == 7)
+      launch_gemm<2, 4, 7>(a, grid, nt, s);
     else
-      k_gemm<2, 4><<<grid, 256, 0, s>>>(a);
-    QW4_LAUNCH_CHECK();
-    if (a.full != nt) {   // the split tiles
-      const int fb = (nt - a.full) * kFixBlocksPerTile;
-      if (variant == 1)
-        k_gemm_fixup<1, 8><<<fb, 64, 0, s>>>(a);
-      else if (variant == 2)
-        k_gemm_fixup<2, 8><<<fb, 64, 0, s>>>(a);
-      else
-        k_gemm_fixup<2, 4><<<fb, 64, 0, s>>>(a);
-    }
+      launch_gemm<2, 4, 8>(a, grid, nt, s);
     QW4_LAUNCH_CHECK();
     return QW4_OK;
   }

@@ -1,0 +1,56 @@
+"""The prefill GEMM's tile heights: 32 to 256 rows per tile (the plan takes the
+height that wastes fewest rows), at the edges of each and in every schedule the
+plan can pick, against the oracle (weights rounded to bf16) on sampled rows,
+bitwise reproducible, and nothing written outside C."""
+import numpy as np
+import pytest
+
+from gpu_util import dev, host, repack_from_logical
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import torch
+
+    assert torch.cuda.is_available(), "GPU test run without a GPU"
+    import w4a16_hip
+
+    w4a16_hip.lib()
+    return w4a16_hip
+
+
+@pytest.fixture(scope="module")
+def ws(hip):
+    w = hip.gemm_workspace_alloc(256 << 20)
+    yield w
+    hip.gemm_workspace_free(w)
+
+
+# one group (fewer than the buffers), a few, a long K; 70 tiles of columns with
+# a ragged last one
+@pytest.mark.parametrize("N,K", [(320, 128), (1024, 640), (5120, 2176), (17856, 1152)])
+def test_gemm_tile_heights(hip, orc, ws, N, K):
+    import torch
+
+    q, zp, s = orc.gen_weights(N, K, seed=N + K)
+    w = repack_from_logical(hip, orc, q, zp, s, "awq_k")
+    for M in (1, 31, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 257, 320, 333, 460,
+              600, 1000):
+        x = orc.gen_x(M, K, seed=M)
+        dx = dev(x)
+        rows = np.unique(np.r_[0, M - 1, M // 2, np.random.default_rng(M).integers(0, M, 3)])
+        ref = orc.matmul_f64(x[rows], q, zp, s, round_w=True)
+        for use in (None, ws):
+            print(f"gemm rows {M} {N}x{K} ws={use is not None}", flush=True)
+            big = torch.full((M + 2, N), 0x5A5A, dtype=torch.int16, device="cuda")
+            hip.gemm_w4a16(big[1:M + 1], w, dx, M, use)
+            again = torch.empty((M, N), dtype=torch.int16, device="cuda")
+            hip.gemm_w4a16(again, w, dx, M, use)
+            torch.cuda.synchronize()
+            assert torch.equal(big[1:M + 1], again)
+            assert (big[0] == 0x5A5A).all() and (big[M + 1] == 0x5A5A).all()
+            m = orc.parity_metrics(host(again, np.uint16)[rows], ref)
+            assert m["max_rel"] <= 1e-2 and m["mean_abs_vs_bf16_ref"] <= 1e-3, (M, m)
+    hip.awq_free(w)
