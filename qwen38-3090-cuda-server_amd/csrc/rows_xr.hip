@@ -328,7 +328,11 @@ bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, hipStream_t st) {
   if (!(2 * a.tiles > cus || (small && a.M >= 8))) return false;
   const int S = fmt == 8 || small ? 1 : 2;
   a.U = a.tiles * 4 / S;
-  a.P = std::max(1, std::min(out == OUT_SWIGLU ? a.U / 2 : a.U, cus));
+  // as few workgroups as give none of them another unit: each brings all rows of
+  // x (34816x5120 at M = 9 / 16: 218 workgroups of 5 units 19.0 / 20.3 us, 256 of 4 or
+  // 5 20.5 / 22.1)
+  const int n = out == OUT_SWIGLU ? a.U / 2 : a.U, most = (n + cus - 1) / cus;
+  a.P = (n + most - 1) / most;
   dispatch(out, fmt, a, S, false, st);
   return true;
 }
