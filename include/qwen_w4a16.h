@@ -238,10 +238,10 @@ int qw4_swiglu(uint16_t* out, const uint16_t* fused, int rows, int inter, void* 
 int qw4_gemv_residual(uint16_t* h, const qw4_weights* w, const uint16_t* x, int M,
                       qw4_scratch* s, void* stream);
 /* linear over the fused [gate | up] weight (out_f = 2 * inter, inter % 64 == 0),
- * then swiglu (model.cu:776-778): y [M][inter]. For M <= 2 (or tmp NULL) the
- * intermediate [M][2 inter] is never written; for M > 2 with tmp
- * ([M][2 inter] bf16) the projection goes through tmp and a separate swiglu,
- * which is faster there. Same results either way. */
+ * then swiglu (model.cu:776-778): y [M][inter]. For M <= 2, without tmp, and
+ * for 2 inter between 8192 and 16384, the intermediate [M][2 inter] is never
+ * written; otherwise with tmp ([M][2 inter] bf16) the projection goes through
+ * tmp and a separate swiglu, which is faster there. Same results either way. */
 int qw4_gemv_swiglu(uint16_t* y, const qw4_weights* w, const uint16_t* x, int M, uint16_t* tmp,
                     qw4_scratch* s, void* stream);
 /* rmsnorm then linear (model.cu:697-700, :773-777): y [M][out_f] = rmsnorm(h) @ W^T

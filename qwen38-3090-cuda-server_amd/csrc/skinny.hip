@@ -746,6 +746,19 @@ __global__ __launch_bounds__(64 * W) void k_dec(SkinnyArgs a) {
       ++lu;
     }
   };
+  // OUT_RES: the residual of the next unit to close (wave 0, lane c: columns 4 c +
+  // st0 ..), loaded a unit ahead: at the close it would cost a memory latency
+  uint32_t resv[(S + 1) / 2];
+  auto load_res = [&](int u) __attribute__((always_inline)) {
+    if (OUT != OUT_RES || wave != 0 || lane >= 16 || u >= u1) return;
+    const uint16_t* r = a.res + (u >> (S == 4 ? 0 : S == 2 ? 1 : 2)) * kTileN + 4 * c + (u % (int)kPer) * S;
+    if (S == 1)
+      resv[0] = r[0];
+    else
+#pragma unroll
+      for (int i = 0; i < S / 2; ++i) resv[i & (S == 1 ? 0 : 1)] = reinterpret_cast<const uint32_t*>(r)[i];
+  };
+  load_res(u0);
   uint32_t* const xw = reinterpret_cast<uint32_t*>(xq);
   if constexpr (OUT != OUT_NORM) {
     // x loads of this wave's groups first (g = wave + W (4 it + lane / 16),
@@ -866,6 +879,23 @@ __global__ __launch_bounds__(64 * W) void k_dec(SkinnyArgs a) {
           emit_swiglu<S>(a, (int)((uint32_t)(u >> 1) / kPer), (int)((uint32_t)(u >> 1) % kPer) * S,
                          gg, uu, lane);
         }
+      } else if (OUT == OUT_RES) {
+        // bf16(res + bf16(acc)), as emit_rows
+        if (lane < 16) {
+          uint32_t o[S];
+#pragma unroll
+          for (int i = 0; i < S; ++i)
+            o[i] = to_bf16(bf16_bits_to_f32((resv[i >> 1] >> (16 * (i & 1))) & 0xffffu) +
+                           bf16_bits_to_f32(to_bf16(t[i])));
+          uint16_t* y = static_cast<uint16_t*>(a.y) + b * kTileN + 4 * c + st0;
+          if (S == 1)
+            y[0] = (uint16_t)o[0];
+          else
+#pragma unroll
+            for (int i = 0; i < S / 2; ++i)
+              reinterpret_cast<uint32_t*>(y)[i] = o[(2 * i) % S] | (o[(2 * i + 1) % S] << 16);
+        }
+        load_res(u + 1);
       } else {
         f32x4 tv[S];
 #pragma unroll
@@ -1189,25 +1219,57 @@ int dec_static_lds(int S, int W) { return 2 * W * S * 16 * 4 + 256; }
 struct DecVariant {
   int S, W, D;
 };
-constexpr DecVariant kDecAll[] = {{2, 8, 3}, {2, 8, 2}, {2, 16, 2}, {2, 8, 4},
-                                  {1, 8, 3}, {1, 16, 3}, {2, 4, 4}, {4, 8, 2}};
-constexpr int kDecPolicy = 3;
+constexpr DecVariant kDecAll[] = {{2, 8, 3}, {2, 8, 2}, {2, 16, 2}, {1, 16, 3},
+                                  {4, 8, 2}, {1, 8, 3}, {2, 8, 4}, {2, 4, 4}};
+constexpr int kDecPolicy = 6;
 constexpr int kDecCount = (int)(sizeof(kDecAll) / sizeof(kDecAll[0]));
 
 // Returns false when the shape does not fit k_dec (activations beyond the
-// per-wave prep, LDS beyond the CU's). Policy, measured on MI355X over the
-// config-2 projections with every variant forced in one process (32-row
-// units throughout; 16-row units and deeper items were slower): when the
-// output has fewer tiles than CUs, 2 items per wave, 16 waves for long K
-// (down: 10.9 us against 11.3 for 8 x 3), 8 for short (qkv: 5.7 against
-// 6.0; o_proj 4.9 against 5.0); else 2 items per wave for short K (32
-// groups) and 8 waves of 3 items otherwise (gate|up).
+// per-wave prep, LDS beyond the CU's). Policy, measured on MI355X with every
+// variant forced in one process. Waves (they fix the order of the sums, so
+// they follow from the shape alone: every epilogue of a shape agrees):
+//  * 16 where the 16-row units all fit one round (4 tiles <= CUs) and K is at
+//    least 32 groups -- few workgroups, bound by the latency of their items: all
+//    three of a wave in flight (896x5120 5.0 -> 4.2 us, 3584x5120 5.3 -> 4.8; at
+//    2048x2048 3.4 against 3.9 for 8 waves);
+//  * 16 of 2 items for K of 64 groups or more and fewer tiles than CUs (down:
+//    10.9 us against 11.3 for 8 x 3);
+//  * else 8, of 2 items for short outputs or K (qkv: 5.7 against 6.0; o_proj 4.9
+//    against 5.0), of 3 otherwise (gate|up).
+// Unit size: 32 rows, but 64 where no workgroup gets more rows for it -- half as
+// many items (8704x5120 7.5 -> 6.7 us, 9600x3200 6.3 -> 5.7). OUT_SWIGLU, whose
+// workgroups own whole (gate, up) pairs: 64 by the same rule (dec_swiglu_rows;
+// 17408x5120 12.7 -> 10.9 us), and 16 where that halves the rows of a single round
+// (4352x5120 7.3 -> 6.5; over several rounds it does not pay: 34816x5120 18.9
+// against 18.3 us for 32-row units, though its fullest workgroup has 160 rows and
+// not 192).
+int dec_swiglu_rows(int tiles, int S, int cus) {
+  const int pairs = tiles / 2 * (4 / S);
+  return (pairs + cus - 1) / cus * 32 * S;
+}
+
 bool dec_config(int out_f, int G, int OUTmode, DecCfg& c) {
   const int tiles = out_f / kTileN;
-  const int K = G * kGroup;
-  DecVariant v = tiles < device_cus() ? (G >= 64 ? kDecAll[2] : kDecAll[1])
-                 : G <= 32            ? kDecAll[1]
-                                      : kDecAll[0];
+  const int K = G * kGroup, cus = device_cus();
+  const bool few = 4 * tiles <= cus && G >= 32;
+  DecVariant v = few            ? kDecAll[3]
+                 : tiles < cus  ? (G >= 64 ? kDecAll[2] : kDecAll[1])
+                 : G <= 32      ? kDecAll[1]
+                                : kDecAll[0];
+  // 64-row units hold more in flight: only where a long K leaves the LDS
+  const bool fits4 = dec_lds_units(K, G, OUTmode == OUT_NORM, 4, 8, 2) * 16 + dec_static_lds(4, 8) <= kLdsBytes;
+  if (v.W == 8) {
+    if (OUTmode == OUT_SWIGLU) {
+      const int r1 = dec_swiglu_rows(tiles, 1, cus), r2 = dec_swiglu_rows(tiles, 2, cus),
+                r4 = dec_swiglu_rows(tiles, 4, cus);
+      if (r4 <= r2 && fits4)
+        v = kDecAll[4];
+      else if (r1 < r2 && 2 * tiles <= cus)
+        v = kDecAll[5];
+    } else if ((tiles + cus - 1) / cus * 64 <= (2 * tiles + cus - 1) / cus * 32 && fits4) {
+      v = kDecAll[4];
+    }
+  }
   if (OUTmode == OUT_BF16 && g_dec_tune.mode.load(std::memory_order_relaxed) == 3) {
     const int tS = g_dec_tune.S.load(std::memory_order_relaxed);
     const int tW = g_dec_tune.W.load(std::memory_order_relaxed);
@@ -1230,10 +1292,13 @@ bool dec_config(int out_f, int G, int OUTmode, DecCfg& c) {
   const int per_wg = c.lds + dec_static_lds(c.S, c.W);
   if (per_wg > kLdsBytes) return false;
   const long long units = (long long)tiles * 4 / c.S;
-  // one workgroup per CU (gate|up: 256 workgroups 17.6 us, two per CU 19.1 us)
+  // one workgroup per CU (gate|up: 256 workgroups 17.6 us, two per CU 19.1 us),
+  // and no more than give none of them another unit (gate|up 218 workgroups of
+  // 5 units 16.6 us, 256 of 4 or 5 17.1; 17408x5120 182 of 3 10.1, 256 of 2 or 3 10.9)
   const long long cap = OUTmode == OUT_SWIGLU ? units / 2 : units;
+  const long long most = (cap + cus - 1) / cus;
   const int tP = g_dec_tune.P.load(std::memory_order_relaxed);
-  c.P = (int)std::max<long long>(1, std::min(cap, tP > 0 ? (long long)tP : (long long)device_cus()));
+  c.P = (int)std::max<long long>(1, tP > 0 ? std::min<long long>(cap, tP) : (cap + most - 1) / most);
   return true;
 }
 
@@ -1678,10 +1743,15 @@ int qw4_gemv_residual(uint16_t* h, const qw4_weights* w, const uint16_t* x, int 
 
 int qw4_gemv_swiglu(uint16_t* y, const qw4_weights* w, const uint16_t* x, int M, uint16_t* tmp,
                     qw4_scratch* s, void* stream) {
-  // Fused for M <= 2; beyond, the pairing of gate and up rows in one
-  // workgroup is slower than the projection plus a separate swiglu (measured
-  // on MI355X), which runs through tmp when one is given.
-  if (M <= 2 || !tmp) return run_skinny<OUT_SWIGLU>(y, w, x, M, s, stream);
+  // Fused for M <= 2, and where the pairs fill one round of workgroups (more
+  // than CUs / 2 tiles, at most CUs: 8704x5120 at M = 9 10.0 us against 12.9, at
+  // 16384x5120 11.7 against 14.2). Elsewhere the pairing of gate and up rows in
+  // one workgroup is no faster than the projection plus a separate swiglu
+  // (17408x5120 16.6 against 16.7, 4352x5120 10.8 against 9.0), which runs through
+  // tmp when one is given.
+  const int tiles = w ? w->out_f / kTileN : 0, cus = device_cus();
+  if (M <= 2 || !tmp || (2 * tiles > cus && tiles <= cus))
+    return run_skinny<OUT_SWIGLU>(y, w, x, M, s, stream);
   if (!w) return QW4_ERR_NULL;
   if (w->out_f % (2 * kTileN)) return QW4_ERR_SHAPE;
   const int st = run_skinny<OUT_BF16>(tmp, w, x, M, s, stream);
