@@ -206,11 +206,28 @@ def _need(t, nbytes: int, where: str) -> None:
             raise ValueError(f"{where}: buffer holds {have} bytes, needs {nbytes}")
 
 
-def _stream(stream) -> int | None:
-    if stream is None:
+_torch = None
+
+
+def _current_stream() -> int:
+    """The calling thread's current stream on its current device. Building
+    torch's Stream object for it takes 3.6 us, the raw handle 0.2 -- of 8.5 us
+    for a whole projection call; before torch has initialized the device, its
+    public call does that first."""
+    global _torch
+    if _torch is None:
         import torch
 
-        return torch.cuda.current_stream().cuda_stream
+        _torch = torch
+    c = _torch._C
+    if _torch.cuda.is_initialized() and hasattr(c, "_cuda_getCurrentRawStream"):
+        return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+    return _torch.cuda.current_stream().cuda_stream
+
+
+def _stream(stream) -> int | None:
+    if stream is None:
+        return _current_stream()
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
