@@ -260,9 +260,9 @@ int qw4_gemv_rmsnorm(uint16_t* y, const qw4_weights* w, const uint16_t* h,
 
 /* ------------------------------------------------------------ dispatch
  * linear() with lin_path() (src/model/model.cu:522-565, :643-658): T rows of
- * x through the GEMV (T = 1), the skinny kernel in chunks of up to 16 rows
- * (2 <= T <= max_t), or the prefill GEMM (T > max_t). max_t is the crossover
- * measured on MI355X for this weight's size (qw4_linear_max_t: 48 rows for
+ * x through the GEMV (T = 1), the skinny kernel in chunks of 16 rows, or 32 in
+ * one pass with the same results (2 <= T <= max_t), or the prefill GEMM (T >
+ * max_t). max_t is the crossover for this weight's size (qw4_linear_max_t: 48 rows for
  * a 93 MB projection, 112 for an 11 MB one); qw4_tune_linear overrides it,
  * as QWEN_MMA_MAX_T does in the reference. ws may be NULL. */
 int qw4_linear(uint16_t* y, const qw4_weights* w, const uint16_t* x, int T, qw4_scratch* s,

@@ -1,5 +1,6 @@
 // k_rows_xr: verify GEMM and heads (M = 2..16) with the activations held in
-// registers, for K up to 8 x kXrMaxGroups groups.
+// registers, for K up to 8 x kXrMaxGroups groups; for K up to 5120 also two
+// 16-row blocks of qw4_linear's small row counts (MB = 2).
 //
 // The work split and the sums are k_rows's (skinny.hip): workgroup p owns whole
 // units (S row quads of a tile over all of K), wave w takes the groups w, w + 8,
@@ -25,12 +26,12 @@ namespace {
 constexpr int kXrW = 8;           // waves
 constexpr int kXrMaxGroups = 8;   // groups a wave can hold: 160 of its 256 registers
 
-// One row m = 4 q + jj of a unit (lane = c + 16 q): columns 64 b + 4 c + st0 + i.
+// One row m = 4 q + m0 of a unit (lane = c + 16 q): columns 64 b + 4 c + st0 + i.
 template <int OUT, int S>
-__device__ __forceinline__ void xr_emit(const SkinnyArgs& a, int b, int st0, int jj,
+__device__ __forceinline__ void xr_emit(const SkinnyArgs& a, int b, int st0, int m0,
                                         const float (&v)[S], const float (&g)[S], int lane,
                                         float& bv, int& bn) {
-  const int c = lane & 15, m = 4 * (lane >> 4) + jj;
+  const int c = lane & 15, m = 4 * (lane >> 4) + m0;
   const int n0 = b * kTileN + 4 * c + st0;
   if (OUT == OUT_ARGMAX) {
 #pragma unroll
@@ -59,17 +60,18 @@ __device__ __forceinline__ void xr_emit(const SkinnyArgs& a, int b, int st0, int
       reinterpret_cast<uint32_t*>(y)[i] = o[2 * i] | (o[2 * i + 1] << 16);
 }
 
-template <int OUT, int FMT, int S, int NG, int D>
+template <int OUT, int FMT, int S, int NG, int D, int MB>
 __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
   using L = DmaSlot<FMT, S>;
   constexpr int W = kXrW;
   constexpr int kL = L::kLoads;
   constexpr uint32_t kPer = 4 / S;
   constexpr uint32_t kQuad = FMT == 8 ? 512u : 256u;
-  // a wave's own area: first the rows of one group on their way into registers
-  // (4 KiB), then its partial sums of a unit, two buffers
-  __shared__ f32x4 red[W][256];
-  static_assert(2 * S * 64 <= 256, "partial sums fit the area");
+  // a wave's own area: first the rows of one group and row block on their way
+  // into registers (4 KiB), then its partial sums of a unit, two buffers
+  constexpr int kArea = 2 * MB * S * 64 > 256 ? 2 * MB * S * 64 : 256;
+  __shared__ f32x4 red[W][kArea];
+  __shared__ f32x4 csum[MB == 1 ? 1 : W][NG][MB][4];   // MB > 1: the row sums (no registers left)
   extern __shared__ u32x4 xr_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, q = lane >> 4;
@@ -88,21 +90,23 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
   const int nw = wave < a.G ? (a.G - 1 - wave) / W + 1 : 0;   // groups of this wave (<= NG)
   const int T = nw * (u1 - u0);                                // its items
 
-  // Activation rows of this wave's groups: load t of a group covers rows 4 t ..
-  // 4 t + 3 whole (1 KiB; rows past M are zeros without traffic, whole loads of
-  // them are not issued).
-  u32x4 x[NG][4];
+  // Activation rows of this wave's groups: load t of a row block covers rows 4 t
+  // .. 4 t + 3 whole (1 KiB; rows past M are zeros without traffic, whole loads
+  // of them are not issued).
+  u32x4 x[NG][MB][4];
   const int xrow = lane >> 4, xch = lane & 15;
 #pragma unroll
   for (int i = 0; i < NG; ++i)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      x[i][t] = u32x4{0u, 0u, 0u, 0u};
-      if (i < nw && 4 * t < a.M)
-        x[i][t] = __builtin_amdgcn_raw_buffer_load_b128(
-            rs.x, (uint32_t)(4 * t + xrow) * (uint32_t)a.K * 2u + (uint32_t)xch * 16u,
-            (uint32_t)(wave + W * i) * 256u, 0);
-    }
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        x[i][mb][t] = u32x4{0u, 0u, 0u, 0u};
+        if (i < nw && 16 * mb + 4 * t < a.M)
+          x[i][mb][t] = __builtin_amdgcn_raw_buffer_load_b128(
+              rs.x, (uint32_t)(16 * mb + 4 * t + xrow) * (uint32_t)a.K * 2u + (uint32_t)xch * 16u,
+              (uint32_t)(wave + W * i) * 256u, 0);
+      }
   __builtin_amdgcn_sched_barrier(0);
 
   // The first D items behind them.
@@ -130,28 +134,37 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
   // row sums with a ones operand, once per group instead of once per item.
   const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u,
                                                        0x3F803F80u, 0x3F803F80u});
-  f32x4 Cs[NG];
+  f32x4 Cs[MB == 1 ? NG : 1];
   {
     u32x4* const area = reinterpret_cast<u32x4*>(red[wave]);
 #pragma unroll
-    for (int i = 0; i < NG; ++i) {
+    for (int i = 0; i < NG; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) area[(4 * t + xrow) * 16 + (xch ^ (4 * t + xrow))] = x[i][t];
-      __builtin_amdgcn_wave_barrier();
+      for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) x[i][t] = area[16 * c + ((4 * q + t) ^ c)];
-      __builtin_amdgcn_wave_barrier();
+        for (int t = 0; t < 4; ++t) area[(4 * t + xrow) * 16 + (xch ^ (4 * t + xrow))] = x[i][mb][t];
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        Cs[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, x[i][t]), ones,
-            t == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : Cs[i], 0, 0, 0);
-    }
+        for (int t = 0; t < 4; ++t) x[i][mb][t] = area[16 * c + ((4 * q + t) ^ c)];
+        __builtin_amdgcn_wave_barrier();
+        f32x4 cs;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          cs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, x[i][mb][t]), ones,
+              t == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : cs, 0, 0, 0);
+        if (MB == 1)
+          Cs[MB == 1 ? i : 0] = cs;
+        else if (c == 0)   // the same for all 16 columns
+          csum[MB == 1 ? 0 : wave][i][mb][q] = cs;
+      }
   }
 
-  f32x4 acc[S];
+  f32x4 acc[MB][S];
 #pragma unroll
-  for (int i = 0; i < S; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int i = 0; i < S; ++i) acc[mb][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float bv = -__builtin_inff();   // OUT_ARGMAX: this thread's best of row m
   int bn = 0x7fffffff;
   float gate[S];                  // OUT_SWIGLU: the gate unit's sums
@@ -172,7 +185,7 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
         wait_items<kL, D>(left - 1);
       RowsData<FMT, S, true> d;
       dma_read<FMT, S, true>(d, ring + j * L::kUnits, lane, st0);
-      f32x4 C[S];
+      f32x4 C[MB][S];
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -184,17 +197,23 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
             const u32x4 v = d.w[i][(t >> 1) & (FMT == 8 ? 1 : 0)];
             B = bytes8_bf16(v[(t & 1) * 2], v[(t & 1) * 2 + 1]);
           }
-          C[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, x[gi][t]), B, t == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : C[i], 0,
-              0, 0);
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            C[mb][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, x[gi][mb][t]), B,
+                t == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : C[mb][i], 0, 0, 0);
         }
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        const uint32_t sbits = (d.s[i >> 1] >> (16 * (S == 1 ? (st0 & 1) : (i & 1)))) & 0xffffu;
-        const float sf = bf16_bits_to_f32(sbits);
-        const float zf = FMT == 4 ? 128.0f + (float)((d.z >> (zsh + 4 * (st0 + i))) & 0xFu) : 128.0f;
+      for (int mb = 0; mb < MB; ++mb) {
+        const f32x4 cs = MB == 1 ? Cs[MB == 1 ? gi : 0] : csum[MB == 1 ? 0 : wave][gi][mb][q];
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) acc[i][jj] += sf * (C[i][jj] - zf * Cs[gi][jj]);
+        for (int i = 0; i < S; ++i) {
+          const uint32_t sbits = (d.s[i >> 1] >> (16 * (S == 1 ? (st0 & 1) : (i & 1)))) & 0xffffu;
+          const float sf = bf16_bits_to_f32(sbits);
+          const float zf = FMT == 4 ? 128.0f + (float)((d.z >> (zsh + 4 * (st0 + i))) & 0xFu) : 128.0f;
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) acc[mb][i][jj] += sf * (C[mb][i][jj] - zf * cs[jj]);
+        }
       }
       // the slot's reads have returned: load the item D ahead into it
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -207,17 +226,20 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
     // a buffer is written again two barriers after it was read.
     const int n = u - u0, par = n & 1;
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-      red[wave][(par * S + i) * 64 + lane] = acc[i];
-      acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        red[wave][((par * MB + mb) * S + i) * 64 + lane] = acc[mb][i];
+        acc[mb][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
     lds_barrier<true>();
-    if ((wave >> 2) == ((OUT == OUT_SWIGLU ? n >> 1 : n) & 1)) {
-      const int jj = wave & 3;
+    // one row block: the halves of the workgroup take turns; two: a half each
+    if (MB == 2 || (wave >> 2) == ((OUT == OUT_SWIGLU ? n >> 1 : n) & 1)) {
+      const int jj = wave & 3, mb = MB == 2 ? wave >> 2 : 0;
       float v[S];
 #pragma unroll
       for (int i = 0; i < S; ++i) {
-        const int at = ((par * S + i) * 64 + lane) * 4 + jj;
+        const int at = (((par * MB + mb) * S + i) * 64 + lane) * 4 + jj;
         v[i] = reinterpret_cast<const float*>(red[0])[at];
 #pragma unroll
         for (int w = 1; w < W; ++w) v[i] += reinterpret_cast<const float*>(red[w])[at];
@@ -227,7 +249,7 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
         for (int i = 0; i < S; ++i) gate[i] = v[i];
       } else {
         const uint32_t ou = OUT == OUT_SWIGLU ? (uint32_t)u >> 1 : (uint32_t)u;   // output unit
-        xr_emit<OUT, S>(a, (int)(ou / kPer), (int)(ou % kPer) * S, jj, v, gate, lane, bv, bn);
+        xr_emit<OUT, S>(a, (int)(ou / kPer), (int)(ou % kPer) * S, 16 * mb + jj, v, gate, lane, bv, bn);
       }
     }
   }
@@ -261,11 +283,11 @@ __global__ __launch_bounds__(64 * kXrW) void k_rows_xr(SkinnyArgs a) {
   }
 }
 
-template <int OUT, int FMT, int S, int NG, int D>
+template <int OUT, int FMT, int S, int NG, int D, int MB = 1>
 void launch(const SkinnyArgs& a, bool prepare, hipStream_t st) {
-  constexpr auto kern = &k_rows_xr<OUT, FMT, S, NG, D>;
+  constexpr auto kern = &k_rows_xr<OUT, FMT, S, NG, D, MB>;
   constexpr int lds = kXrW * D * DmaSlot<FMT, S>::kUnits * 16;
-  static_assert(lds + kXrW * 4096 <= kLdsBytes, "ring and areas fit the CU's LDS");
+  static_assert(lds + kXrW * (MB * 4096 + NG * MB * 64) <= kLdsBytes, "ring and areas fit the CU's LDS");
   allow_lds<kern>(lds);
   if (!prepare) kern<<<a.P, 64 * kXrW, lds, st>>>(a);
 }
@@ -337,8 +359,28 @@ bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, hipStream_t st) {
   return true;
 }
 
+// Two row blocks (17 to 32 rows of qw4_linear) in one pass, each bitwise what a
+// pass of its own gives, for K up to 5120 (32 registers a group: 230 in all, no
+// spills). Faster than two passes at every size measured (32 rows): gate|up
+// 34816x5120 40.0 -> 27.5 us, 7168x5120 15.5 -> 11.4, 5120x4096 12.9 -> 10.3,
+// 896x5120 12.3 -> 10.8, 5120x512 7.9 -> 6.0.
+bool rows_xr2_launch(SkinnyArgs& a, int cus, hipStream_t st) {
+  const int ng = (a.G + kXrW - 1) / kXrW;
+  if (a.M < 17 || a.M > 32 || ng > 5) return false;
+  a.U = a.tiles * 2;
+  const int most = (a.U + cus - 1) / cus;
+  a.P = (a.U + most - 1) / most;
+  if (ng <= 3)
+    launch<OUT_BF16, 4, 2, 3, 3, 2>(a, false, st);
+  else
+    launch<OUT_BF16, 4, 2, 5, 3, 2>(a, false, st);
+  return true;
+}
+
 void rows_xr_prepare() {
   SkinnyArgs a{};
+  launch<OUT_BF16, 4, 2, 3, 3, 2>(a, true, nullptr);
+  launch<OUT_BF16, 4, 2, 5, 3, 2>(a, true, nullptr);
   dispatch(0, 4, a, 0, true, nullptr);
   dispatch(0, 8, a, 0, true, nullptr);
 }

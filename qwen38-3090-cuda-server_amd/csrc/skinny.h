@@ -519,6 +519,11 @@ void allow_lds(int bytes) {
 // k_rows_xr (rows_xr.hip): launches it for these arguments (P and U filled in)
 // and returns true, or returns false where it does not apply.
 bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, hipStream_t st);
+bool rows_xr2_launch(SkinnyArgs& a, int cus, hipStream_t st);   // 17 to 32 rows
+// qw4_linear's 17 to 32 rows over one reading of the weights, each bitwise a
+// 16-row pass's (skinny.hip); *taken false where that form does not apply.
+int skinny_rows32(uint16_t* y, const qw4_weights* w, const uint16_t* x, int M, qw4_scratch* s,
+                  void* stream, bool* taken);
 void rows_xr_prepare();   // raises its kernels' dynamic LDS limits on this device
 
 }  // namespace qw4

@@ -1623,6 +1623,36 @@ int noalloc_scratch(uint64_t*& ptr) {
 
 using namespace qw4;
 
+// qw4_linear's pass of 17 to 32 rows over one reading of the weights: the checks of qw4_gemm_small, then k_rows_xr with two row blocks.
+int qw4::skinny_rows32(uint16_t* y, const qw4_weights* w, const uint16_t* x, int M, qw4_scratch* s,
+                       void* stream, bool* taken) {
+  *taken = false;
+  int st = check_weights_public(w);
+  if (st) return st;
+  if (!y || !x || !s || !s->counters || !s->keys) return QW4_ERR_NULL;
+  if (((uintptr_t)x & 15) || ((uintptr_t)y & 7)) return QW4_ERR_ALIGN;
+  const int tiles = w->out_f / kTileN;
+  if (tiles > s->max_tiles || s->max_m < 16 || w->in_f > s->max_in) return QW4_ERR_SCRATCH;
+  const size_t weight_bytes = (size_t)w->out_f * w->in_f / 2;
+  if (weight_bytes >= (1ull << 32)) return QW4_ERR_SHAPE;
+  if (g_dec_tune.mode.load(std::memory_order_relaxed) != 0) return QW4_OK;
+  SkinnyArgs a{};
+  a.qw = w->qweight;
+  a.sc = w->scale;
+  a.zr = w->zeros;
+  a.x = x;
+  a.y = y;
+  a.M = M;
+  a.N = a.ld = w->out_f;
+  a.K = w->in_f;
+  a.G = w->num_groups;
+  a.tiles = tiles;
+  a.weight_bytes = (uint32_t)weight_bytes;
+  *taken = rows_xr2_launch(a, device_cus(), (hipStream_t)stream);
+  if (*taken) QW4_LAUNCH_CHECK();
+  return QW4_OK;
+}
+
 extern "C" {
 
 int qw4_tune_decode(int mode, int S, int W, int D, int P) {
