@@ -84,7 +84,9 @@ constexpr int kRowsXmChunks = 16;
 // only those lanes take part in the unit sums and only that element is
 // accumulated; without (M > 1) each item's activations still go to registers,
 // loaded with the item.
-template <int OUT, int FMT, int S, int W, bool XL, int D, bool DMA = false, bool XM = false>
+// X4: all four activation loads per item (M > 12), their number known.
+template <int OUT, int FMT, int S, int W, bool XL, int D, bool DMA = false, bool XM = false,
+          bool X4 = true>
 __global__ __launch_bounds__(64 * W) void k_rows(SkinnyArgs a) {
   // LDS-DMA items with staged activations: M = 1, or (XM) M > 1 with each
   // activation row padded by one 16-byte chunk, so that the 16 lanes reading
@@ -148,6 +150,7 @@ __global__ __launch_bounds__(64 * W) void k_rows(SkinnyArgs a) {
   // !XL: lane l of activation load t fetches row 4 t + l / 16, chunk
   // (l % 16) ^ row, into slot unit 64 t + l (see rows_slot_units)
   const int xr_ = lane >> 4, xj_ = lane & 15;
+  const int nx = X4 ? 4 : (a.M + 3) / 4;   // activation loads of an item
   uint32_t xdoff[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -163,10 +166,20 @@ __global__ __launch_bounds__(64 * W) void k_rows(SkinnyArgs a) {
                       in ? (uint32_t)b * (uint32_t)a.G + (uint32_t)g : oob_blk,
                       wbase + (uint32_t)st0 * kQuad, lane);
     if (!XL) {
+      // loads whose four rows all lie past M are not issued (a zero-filled load
+      // holds the address unit as long as a real one:
+      // 5120x8704 at M = 2 / 5 / 9 9.4 / 10.2 / 11.0 -> 9.0 / 9.9 / 10.7 us); what
+      // their place in the slot holds only reaches output rows that are never
+      // stored.
       u32x4* const xs = ring + j * kSlotU + DmaSlot<FMT, S>::kUnits;
+      if (nx == 4) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        dma_load16c(rs.x, xs + 64 * t, xdoff[t], (uint32_t)g * 256u);
+        for (int t = 0; t < 4; ++t) dma_load16c(rs.x, xs + 64 * t, xdoff[t], (uint32_t)g * 256u);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+          if (t < nx) dma_load16c(rs.x, xs + 64 * t, xdoff[t], (uint32_t)g * 256u);
+      }
     }
     lg += W;
     if (lg >= a.G) {
@@ -314,13 +327,31 @@ __global__ __launch_bounds__(64 * W) void k_rows(SkinnyArgs a) {
   if constexpr (DMA) {
     // item t waits for its slot; the loads of the items after it (all D - 1
     // of them in the main loop, fewer in the tail) may still be in flight
-    constexpr int kL = DmaSlot<FMT, S>::kLoads + (XL ? 0 : 4);
+    // (nc: the number of those items, -1 if only known at run time, in nwait)
+    constexpr int kL = DmaSlot<FMT, S>::kLoads;
     auto step_dma = [&](auto jc, auto nc, bool reload, int nwait = 0) __attribute__((always_inline)) {
       constexpr int j = decltype(jc)::value;
-      if constexpr (decltype(nc)::value >= 0)
-        wait_vm<decltype(nc)::value>();
-      else
-        wait_items<kL, D>(nwait);
+      constexpr int n = decltype(nc)::value;
+      if constexpr (XL) {
+        if constexpr (n >= 0)
+          wait_vm<(n < 0 ? 0 : n) * kL>();
+        else
+          wait_items<kL, D>(nwait);
+      } else {
+        auto wait_x = [&](auto xc) __attribute__((always_inline)) {   // x activation loads per item
+          constexpr int x = decltype(xc)::value;
+          if constexpr (n >= 0)
+            wait_vm<(n < 0 ? 0 : n) * (kL + x)>();
+          else
+            wait_items<kL + x, D>(nwait);
+        };
+        if (nx == 4)
+          wait_x(std::integral_constant<int, 4>{});
+        else
+          static_for<1, 4>([&](auto xc) {
+            if (nx == decltype(xc)::value) wait_x(xc);
+          });
+      }
       const int st0 = (int)((uint32_t)real_unit(closed) % kPer) * S;
       RowsData<FMT, S, XL> d;
       dma_read<FMT, S, XL>(d, ring + j * kSlotU, lane, st0);
@@ -348,7 +379,7 @@ __global__ __launch_bounds__(64 * W) void k_rows(SkinnyArgs a) {
     // the last item: an out-of-range LDS-DMA load costs as much as a real one)
     for (; t0 + 2 * D <= T; t0 += D)
       static_for<0, D>([&](auto jc) {
-        step_dma(jc, std::integral_constant<int, (D - 1) * kL>{}, true);
+        step_dma(jc, std::integral_constant<int, D - 1>{}, true);
       });
     const int r = T - t0;
     static_for<0, 2 * D - 1>([&](auto jc) {
@@ -1334,14 +1365,23 @@ void prepare_dec() {
 template <int OUT, int FMT, int S, int W, int D, bool XL, bool XM = false>
 void launch_rows_dma_d(const SkinnyArgs& a, hipStream_t st) {
   const int lds = (XL ? a.M * (a.K * 2 + (XM ? 16 : 0)) : 0) + W * D * rows_slot_units<FMT, S, XL>() * 16;
+  if constexpr (!XL) {
+    if (a.M <= 12) {
+      constexpr auto few = &k_rows<OUT, FMT, S, W, XL, D, true, XM, false>;
+      allow_lds<few>(lds);
+      few<<<a.P, 64 * W, lds, st>>>(a);
+      return;
+    }
+  }
   constexpr auto kern = &k_rows<OUT, FMT, S, W, XL, D, true, XM>;
   allow_lds<kern>(lds);
   kern<<<a.P, 64 * W, lds, st>>>(a);
 }
 
-template <int OUT, int FMT, int S, bool XL, int D, bool XM = false>
+template <int OUT, int FMT, int S, bool XL, int D, bool XM = false, bool X4 = true>
 void prepare_dma_one() {
-  constexpr auto kern = &k_rows<OUT, FMT, S, 8, XL, D, true, XM>;
+  if constexpr (!XL && X4) prepare_dma_one<OUT, FMT, S, XL, D, XM, false>();
+  constexpr auto kern = &k_rows<OUT, FMT, S, 8, XL, D, true, XM, X4>;
   hipFuncAttributes at{};
   if (hipFuncGetAttributes(&at, reinterpret_cast<const void*>(kern)) == hipSuccess)
     allow_lds<kern>(kLdsBytes - (int)at.sharedSizeBytes);
