@@ -144,8 +144,10 @@ int qw4_tune_decode(int mode, int S, int W, int D, int P);
  * workgroup per tile, 1 stream-K, 2 hybrid, 3 split-K (every tile cut into the
  * same k-slices; at most CUs / 2 tiles) (split schedules need a workspace);
  * variant 0 the default kernel (4 waves, each on a whole 64-row weight tile
- * against all 256 activation rows), 1 8 waves on 32-row tile halves, 2 8 waves
- * on whole tiles against 128 rows; the variants' results are bitwise equal. */
+ * against all activation rows of the workgroup's tile, 32 to 256), 1 8 waves
+ * on 32-row tile halves, 2 8 waves on whole tiles against half the rows (both
+ * computing 256 rows whatever the tile's); under every schedule the variants'
+ * results are bitwise equal. */
 int qw4_tune_gemm(int schedule, int variant);
 /* qw4_tune_linear: max_t of qw4_linear for every weight, 0 = the measured rule
  * (the role of the reference's QWEN_MMA_MAX_T environment variable). */

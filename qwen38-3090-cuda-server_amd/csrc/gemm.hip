@@ -64,6 +64,7 @@ struct GemmArgs {
   uint16_t* C;
   float* slots;         // stream-K: [P][2] fp32 partial tiles
   int M, N, K, G, tiles_n, tiles_m, map;
+  int bm;               // rows of a tile (8-wave variants; 32 MB in the default kernels)
   int P;                // workgroups
   // map: 0 blockIdx order; 1 XCD-contiguous runs of workgroups; 2 split-K:
   // XCD-contiguous runs over (k-slice, tile row-major), P / tiles slices
@@ -288,6 +289,19 @@ __device__ __forceinline__ void g2_group(const GemmArgs& a, f32x16v (&acc)[NH][G
   }
 }
 
+// Rows of a tile. The 8-wave variants exist for MB = 8 only and run the plan's
+// lower tiles in it (rows past bm read as zeros and are not stored), so that a
+// call is cut the same way under every variant.
+template <int NW, int MB>
+__device__ __forceinline__ int g2_tile_rows(const GemmArgs& a) {
+  return NW == 8 ? a.bm : 32 * MB;
+}
+// First row past the tile at m0 that is not stored.
+template <int NW>
+__device__ __forceinline__ int g2_row_end(const GemmArgs& a, int m0) {
+  return NW == 8 ? min(a.M, m0 + a.bm) : a.M;
+}
+
 // One wave's share of one (tile, group range) segment: acc = sum over groups
 // [g0, g1) of this wave's weight rows x the tile's activation rows.
 template <int NH, int NW, int MB>
@@ -303,10 +317,10 @@ __device__ __forceinline__ void g2_segment(const GemmArgs& a, const G2Rsrc& rs,
   for (int j = 0; j < NH; ++j)
 #pragma unroll
     for (int mb = 0; mb < MBW; ++mb) acc[j][mb] = f32x16v{};
-  // Activation rows [m0, M): the buffer's end turns rows past M into zeros.
+  // Activation rows [m0, row end): the buffer's end turns rows past it into zeros.
   const uint32_t row_bytes = (uint32_t)a.K * 2u;
   const __amdgpu_buffer_rsrc_t act = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(a.A) + (size_t)m0 * a.K, 0, (int)((uint32_t)(a.M - m0) * row_bytes),
+      const_cast<uint16_t*>(a.A) + (size_t)m0 * a.K, 0, (int)((uint32_t)(g2_row_end<NW>(a, m0) - m0) * row_bytes),
       0x00020000);
   const __amdgpu_buffer_rsrc_t act_none =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.A), 0, 0, 0x00020000);
@@ -413,7 +427,7 @@ __device__ __forceinline__ void g2_store_staged(const GemmArgs& a,
     const int row = RPI * t + lane / CPR;
     const u32x4 v = reg[row * CPR + (cl ^ (row % CPR))];
     const int m = m0 + 32 * mw + row;
-    if (m < a.M)
+    if (m < g2_row_end<NW>(a, m0))
       *reinterpret_cast<u32x4*>(a.C + (size_t)m * a.N + tile * kTileN + 32 * b0 + 8 * cl) = v;
   }
 }
@@ -530,12 +544,12 @@ __global__ __launch_bounds__(64) void k_gemm_fixup(GemmArgs a) {
     }
   }
   // pair index j * MBW + mb (g2_slot_store's order)
-  const int m0 = tm * 32 * MB;
+  const int m0 = tm * g2_tile_rows<NW, MB>(a);
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
     const int idx = part * kPer + e, j = idx / MBW, mb = idx % MBW;
     const int m = m0 + 32 * (mw + mb) + r;
-    if (m >= a.M) continue;
+    if (m >= g2_row_end<NW>(a, m0)) continue;
     uint16_t* crow = a.C + (size_t)m * a.N + tile * kTileN;
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
@@ -550,8 +564,8 @@ template <int NH, int NW, int MB>
 __global__ __launch_bounds__(64 * NW, 1) void k_gemm(GemmArgs a) {
   using Sp = G2Split<NH, NW, MB>;
   constexpr int MBW = Sp::MBW;              // m-blocks per wave
-  constexpr int BM = 32 * MB;               // rows of a tile
-  __shared__ u32x4 lds[Sp::DEPTH][BM * 16];   // [row][16 swizzled chunks]
+  const int bm = g2_tile_rows<NW, MB>(a);   // rows of a tile
+  __shared__ u32x4 lds[Sp::DEPTH][32 * MB * 16];   // [row][16 swizzled chunks]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform
   const int lane = threadIdx.x & 63;
   int wt, b0, mw;
@@ -590,8 +604,8 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm(GemmArgs a) {
     const int tile = tn * 4 + wt;
     const bool valid = tile * kTileN < a.N;
     const int ltile = valid ? tile : (a.N / kTileN - 1);
-    g2_segment<NH, NW, MB>(a, wr, lds, acc, tm * BM, ltile, b0, mw, 0, a.G, wave, lane);
-    g2_store_staged<NH, NW, MB>(a, acc, &lds[0][0], tm * BM, tile, b0, mw, valid, wave, lane);
+    g2_segment<NH, NW, MB>(a, wr, lds, acc, tm * bm, ltile, b0, mw, 0, a.G, wave, lane);
+    g2_store_staged<NH, NW, MB>(a, acc, &lds[0][0], tm * bm, tile, b0, mw, valid, wave, lane);
   }
   for (int u = u0; u < u1;) {
     const int ts = u / a.G, g0 = u - ts * a.G;
@@ -601,9 +615,9 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm(GemmArgs a) {
     const int tile = tn * 4 + wt;
     const bool valid = tile * kTileN < a.N;
     const int ltile = valid ? tile : (a.N / kTileN - 1);
-    g2_segment<NH, NW, MB>(a, wr, lds, acc, tm * BM, ltile, b0, mw, g0, g1, wave, lane);
+    g2_segment<NH, NW, MB>(a, wr, lds, acc, tm * bm, ltile, b0, mw, g0, g1, wave, lane);
     if (g0 == 0 && g1 == a.G) {
-      g2_store_staged<NH, NW, MB>(a, acc, &lds[0][0], tm * BM, tile, b0, mw, valid, wave, lane);
+      g2_store_staged<NH, NW, MB>(a, acc, &lds[0][0], tm * bm, tile, b0, mw, valid, wave, lane);
     } else {
       g2_slot_store<NH, NW, MB>(rs, acc, vp, u == u0 ? 0 : 1, wave, lane);
     }
@@ -633,8 +647,8 @@ int device_cus() {
 std::atomic<int> g_gemm_schedule{-1};
 // Kernel variant (qw4_tune_gemm): 0 the default, 4 waves of whole 64-row
 // tiles against all 256 activation rows; 1 8 waves of 32-row tile halves; 2 8
-// waves of whole tiles against 128 rows. All three sum every output in the
-// same order, so their results are bitwise equal.
+// waves of whole tiles against 128 rows. All three cut a call the same way and
+// sum every output in the same order, so their results are bitwise equal.
 std::atomic<int> g_gemm_variant{0};
 
 template <int NH, int NW, int MB>
@@ -762,14 +776,14 @@ int qw4_gemm(uint16_t* C, const qw4_weights* w, const uint16_t* A, int M, qw4_wo
     // 66, o 5120x4096 36 / 36 / 40 -> 19 / 23 / 31), and few tiles, cut in fewer
     // slices (o at 256 rows 37 -> 28). By 3% at least, what the model resolves:
     // down at 2000 rows costs 100.9 in 224-row tiles against 101.3 and is 3% slower.
-    if (schedule == -1 && variant == 0)
+    if (schedule == -1)
       for (int mb = 7; mb >= 2; --mb) {
         const GemmPlan q = gemm_plan(M, w->out_f, w->num_groups, mb, cus, ws_ok, schedule);
         if (q.cost < 0.97 * p.cost) p = q;
       }
     const int nt = p.tiles_n * p.tiles_m, mb = p.mb;
     GemmArgs a{w->qweight, w->scale, w->zeros, A, C, nullptr, M, w->out_f, w->in_f,
-                w->num_groups, p.tiles_n, p.tiles_m, nt % 8 == 0, nt, nt, 0};
+                w->num_groups, p.tiles_n, p.tiles_m, nt % 8 == 0, 32 * mb, nt, nt, 0};
     int grid = nt;
     if (p.pick == 3) {
       a.slots = static_cast<float*>(ws->buf);

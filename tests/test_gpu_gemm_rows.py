@@ -54,3 +54,39 @@ def test_gemm_tile_heights(hip, orc, ws, N, K):
             m = orc.parity_metrics(host(again, np.uint16)[rows], ref)
             assert m["max_rel"] <= 1e-2 and m["mean_abs_vs_bf16_ref"] <= 1e-3, (M, m)
     hip.awq_free(w)
+
+
+# split-K with other slices than 256-row tiles have, stream-K, hybrid and whole
+# tiles, all below 256 rows a tile; ragged last rows and columns
+@pytest.mark.parametrize("M,N,K", [(200, 1024, 2560), (200, 5120, 4096), (333, 5184, 2176),
+                                   (100, 34816, 5120), (300, 34816, 5120), (300, 34816, 1024)])
+def test_gemm_variants_bitwise_at_the_plan(hip, ws, M, N, K):
+    """Under the cost model's own schedule (-1) too, the kernel variants cut a call
+    the same way: bitwise equal, and nothing written outside C."""
+    import torch
+
+    G = K // 128
+    q = torch.empty(K // 8 * N, dtype=torch.int32, device="cuda")
+    s = torch.empty(G * N, dtype=torch.int16, device="cuda")
+    z = torch.empty(G * N // 8, dtype=torch.int32, device="cuda")
+    hip.gen_awq_k(q, s, z, N, K, N + K, 3)
+    w = hip.awq_alloc_fused(N, K)
+    hip.awq_repack_awq_into(w, 0, q, s, z, N, hip.LAYOUT_AWQ_K)
+    x = torch.empty(M * K, dtype=torch.int16, device="cuda")
+    hip.gen_bf16(x, M * K, 0, M + K, 0)
+    try:
+        for use in (None, ws):
+            outs = []
+            for variant in (0, 1, 2):
+                print(f"gemm variant {variant} {M}x{N}x{K} ws={use is not None}", flush=True)
+                hip.tune_gemm(-1, variant)
+                big = torch.full((M + 2, N), 0x5A5A, dtype=torch.int16, device="cuda")
+                hip.gemm_w4a16(big[1:M + 1], w, x, M, use)
+                outs.append(big)
+            torch.cuda.synchronize()
+            assert (outs[0][0] == 0x5A5A).all() and (outs[0][M + 1] == 0x5A5A).all()
+            for variant in (1, 2):
+                assert torch.equal(outs[0], outs[variant]), variant
+    finally:
+        hip.tune_gemm(-1, 0)
+    hip.awq_free(w)
