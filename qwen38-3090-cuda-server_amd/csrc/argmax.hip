@@ -37,16 +37,14 @@ __device__ __forceinline__ float ldbf(const uint16_t* p) { return bf16_bits_to_f
 // (-FLT_MAX, 0) and takes a value only if strictly greater, so the lowest index
 // wins ties and values never above -FLT_MAX (or NaN) leave index 0.
 //
-// One workgroup per row (the entry point has no scratch to combine several),
-// so a row is bound by what one CU keeps in flight: 16 waves with kRowChunks
-// 16-byte loads each (128 KiB). A chunk of 8 values costs a max tree and one
-// compare; the place inside the chunk is looked up once, for the thread's best
-// chunk. 5 rows of 248320 logits: 261 us with 256
-// threads and 2-byte loads, 12 us so (head and argmax together 486 -> 237 us).
-constexpr int kRowThreads = 1024;
+// One workgroup of T threads per row (the entry point has no scratch to combine
+// several), so a row is bound by what one workgroup keeps in flight: kRowChunks
+// 16-byte loads a thread. A chunk of 8 values costs a max tree and one compare;
+// the place inside the chunk is looked up once, for the thread's best chunk.
 constexpr int kRowChunks = 8;
 
-__global__ __launch_bounds__(kRowThreads) void k_argmax_rows(int32_t* out, const uint16_t* x, int n) {
+template <int T>
+__global__ __launch_bounds__(T) void k_argmax_rows(int32_t* out, const uint16_t* x, int n) {
   const uint16_t* row = x + (size_t)blockIdx.x * n;
   float v = -FLT_MAX;
   int i = 0;
@@ -61,20 +59,22 @@ __global__ __launch_bounds__(kRowThreads) void k_argmax_rows(int32_t* out, const
   if ((int)threadIdx.x < head) take(threadIdx.x);
   const u32x4* body = reinterpret_cast<const u32x4*>(row + head);
   int best = -1;   // the chunk that holds this thread's best value
-  for (int k = threadIdx.x; k < chunks; k += kRowChunks * kRowThreads) {
+  for (int k = threadIdx.x; k < chunks; k += kRowChunks * T) {
+    const int left = chunks - (k - (int)threadIdx.x);   // chunks of the row from this round on
     u32x4 d[kRowChunks];
 #pragma unroll
     for (int j = 0; j < kRowChunks; ++j) {
-      const int kj = k + j * kRowThreads;
-      d[j] = body[kj < chunks ? kj : k];   // past the end: chunk k again, never greater
+      const int kj = k + j * T;
+      if (j * T < left) d[j] = body[kj < chunks ? kj : k];   // past the end: chunk k again, never greater
     }
 #pragma unroll
     for (int j = 0; j < kRowChunks; ++j) {
+      if (j * T >= left) break;   // uniform: a short row has fewer rounds of loads
       float m = -FLT_MAX;   // fmaxf passes over NaN
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         m = fmaxf(m, fmaxf(__uint_as_float(d[j][e] << 16), __uint_as_float(d[j][e] & 0xffff0000u)));
-      if (m > v) { v = m; best = k + j * kRowThreads; }
+      if (m > v) { v = m; best = k + j * T; }
     }
   }
   if (best >= 0) {
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kRowThreads) void k_argmax_rows(int32_t* out, const
   }
   const int tail = head + 8 * chunks + (int)threadIdx.x;
   if (tail < n) take(tail);
-  block_best<kRowThreads / 64>(v, i);
+  block_best<T / 64>(v, i);
   if (threadIdx.x == 0) out[blockIdx.x] = i;
 }
 
@@ -134,7 +134,20 @@ int qw4_argmax_rows(int32_t* out, const uint16_t* x, int rows, int n, void* stre
   if (!out || !x) return QW4_ERR_NULL;
   if (rows < 0 || n <= 0) return QW4_ERR_SHAPE;
   if (rows == 0) return QW4_OK;
-  k_argmax_rows<<<rows, kRowThreads, 0, (hipStream_t)stream>>>(out, x, n);
+  // Few long rows: 16 waves a row, for what one CU can keep in flight (5 rows of
+  // 248320: 116 us with 256 threads and 2-byte loads, 25 with 256 threads and
+  // 16-byte loads, 14 so; at 24000 values 256 and 1024 threads meet). Short rows:
+  // the waves of a workgroup are the cost (16384 rows of 64: 1024 threads 80 us, 256
+  // 17, 64 8; of 1000: 83, 20, 10; from 4096 values on 256 beat 64). More rows than
+  // two a CU need no 16 waves each to fill it (1000 rows of 64000: 31 us, 256
+  // threads 25).
+  hipStream_t hs = (hipStream_t)stream;
+  if (n > 24576 && rows <= 512)
+    k_argmax_rows<1024><<<rows, 1024, 0, hs>>>(out, x, n);
+  else if (n > 2048)
+    k_argmax_rows<256><<<rows, 256, 0, hs>>>(out, x, n);
+  else
+    k_argmax_rows<64><<<rows, 64, 0, hs>>>(out, x, n);
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }

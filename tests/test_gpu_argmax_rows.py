@@ -45,3 +45,22 @@ def test_argmax_rows(orc, n, kind):
     assert np.array_equal(got, _strict_argmax(v))
     if kind != "special":
         assert np.array_equal(got, orc.argmax_rows_bf16(v))
+
+
+# the edges of the workgroup sizes: 64 threads up to 2048 values, 1024 for rows of
+# more than 24576 values in calls of at most 512 rows, 256 for the others
+@pytest.mark.parametrize("n,rows", [(2047, 300), (2048, 3), (2049, 300), (24576, 5), (24577, 5),
+                                    (24583, 512), (24583, 513), (3, 70000)])
+def test_argmax_rows_workgroups(orc, n, rows):
+    import torch
+    import w4a16_hip as hip
+
+    v = orc.gen_x(rows, n, seed=n + rows)
+    v[0, -1] = v[rows - 1, 0] = 0x7F80          # +inf: the last and the first place
+    out = empty((rows + 1,), np.int32)
+    out.fill_(-7)
+    print(f"argmax rows n={n} rows={rows}", flush=True)
+    hip.argmax_rows(out[:rows], dev(v), rows, n)
+    torch.cuda.synchronize()
+    got = host(out, np.int32)
+    assert np.array_equal(got[:rows], _strict_argmax(v)) and got[rows] == -7
