@@ -24,31 +24,32 @@ constexpr int kEwThreads = 256;
 // kept for the output, so a row costs one memory latency. Rows of 5120, us: 1 row
 // 3.5 -> 2.3, 200 4.5 -> 3.0 (T = 1024); 1000 7.7 -> 7.1, 4096 21.5 -> 17.9 (T = 256;
 // 1024 threads take 7.7 and 21.6 there).
-template <int T>
+// PER: the chunks a thread keeps, kNormVThreads / T or as few as hold the row.
+template <int T, int PER>
 __global__ __launch_bounds__(T) void k_rmsnorm(uint16_t* __restrict__ out,
                                                const uint16_t* __restrict__ x,
                                                const uint16_t* __restrict__ w, int dim, float eps) {
-  constexpr int kPer = kNormVThreads / T;
   const int row = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int kc = dim / 8;
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + (size_t)row * dim);
   const u32x4* wr = reinterpret_cast<const u32x4*>(w);
   u32x4* orow = reinterpret_cast<u32x4*>(out + (size_t)row * dim);
   __shared__ float vsum[kNormVWaves];
-  u32x4 xv[kPer], wv[kPer];
+  u32x4 xv[PER], wv[PER];
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
+  for (int k = 0; k < PER; ++k) {
     const int i = min(t + T * k, kc - 1);
     xv[k] = xr[i];
     wv[k] = wr[i];
   }
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
+  for (int k = 0; k < PER; ++k) {
     float ss = t + T * k < kc ? norm_sumsq(0.f, xv[k]) : 0.f;
     for (int i = t + T * k + kNormVThreads; i < kc; i += kNormVThreads) ss = norm_sumsq(ss, xr[i]);
     ss = norm_wave_sum(ss);
     if (lane == 0) vsum[wave + (T / 64) * k] = ss;
   }
+  if (t < kNormVWaves - PER * (T / 64)) vsum[PER * (T / 64) + t] = 0.f;   // virtual waves past the row
   __syncthreads();
   const float inv = norm_inv(vsum, dim, eps);
   auto store = [&](int i, const u32x4& v, const u32x4& g) {
@@ -59,7 +60,7 @@ __global__ __launch_bounds__(T) void k_rmsnorm(uint16_t* __restrict__ out,
     orow[i] = o;
   };
 #pragma unroll
-  for (int k = 0; k < kPer; ++k)
+  for (int k = 0; k < PER; ++k)
     if (t + T * k < kc) store(t + T * k, xv[k], wv[k]);
   for (int i = t + kNormVThreads; i < kc; i += T) store(i, xr[i], wr[i]);
 }
@@ -119,11 +120,19 @@ int qw4_rmsnorm(uint16_t* out, const uint16_t* x, const uint16_t* w, int rows, i
   if (((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) & 15) return QW4_ERR_ALIGN;
   if (rows == 0) return QW4_OK;
   // few rows: one virtual thread per thread, for latency; from about two
-  // workgroups of 1024 per CU on, smaller workgroups balance better
+  // workgroups of 1024 per CU on, smaller workgroups balance better. Those load
+  // as many rounds of chunks as a row has, up to the four of the virtual threads:
+  // with four for every row, 16384 rows of 128 / 1024 / 2048 took 25.3 / 28.4 / 30.8 us,
+  // 12.0 / 15.7 / 21.7 so.
+  hipStream_t hs = (hipStream_t)stream;
   if (rows <= 512)
-    k_rmsnorm<kNormVThreads><<<rows, kNormVThreads, 0, (hipStream_t)stream>>>(out, x, w, dim, eps);
+    k_rmsnorm<kNormVThreads, 1><<<rows, kNormVThreads, 0, hs>>>(out, x, w, dim, eps);
+  else if (dim <= 8 * kEwThreads)
+    k_rmsnorm<kEwThreads, 1><<<rows, kEwThreads, 0, hs>>>(out, x, w, dim, eps);
+  else if (dim <= 16 * kEwThreads)
+    k_rmsnorm<kEwThreads, 2><<<rows, kEwThreads, 0, hs>>>(out, x, w, dim, eps);
   else
-    k_rmsnorm<kEwThreads><<<rows, kEwThreads, 0, (hipStream_t)stream>>>(out, x, w, dim, eps);
+    k_rmsnorm<kEwThreads, 4><<<rows, kEwThreads, 0, hs>>>(out, x, w, dim, eps);
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }

@@ -1,6 +1,6 @@
 """rmsnorm at the edges of its two workgroup sizes (1024 threads up to 512 rows,
-256 beyond) and of the chunks a thread keeps (rows up to 8192 values): one
-chunk, a row shorter than a workgroup, exactly 8192, one chunk more, several
+256 beyond) and of the chunks a thread keeps (one, two or four rounds of 256:
+rows up to 2048, 4096 and 8192 values): one chunk, a row shorter than a workgroup, exactly 8192, one chunk more, several
 rounds. Rows do not depend on the workgroup size: bitwise the same row in a
 call of 512 and of 513 rows."""
 import numpy as np
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 EPS = 1e-6
 
 
-@pytest.mark.parametrize("dim", [8, 1000, 2056, 8192, 8200, 17408])
+@pytest.mark.parametrize("dim", [8, 1000, 2048, 2056, 4096, 4104, 8192, 8200, 17408])
 def test_rmsnorm_rows(orc, dim):
     import torch
 
