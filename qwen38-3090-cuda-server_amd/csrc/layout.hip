@@ -123,29 +123,33 @@ __global__ __launch_bounds__(256) void k_repack(uint32_t* __restrict__ dst,
 
 // ----------------------------------------------------------------- dequant
 // dst [nrows][K] = RNE(float(q - z) * s). One workgroup per (tile, kDeqGroups
-// groups), so a block's lines are read by one CU and every 16 lanes write 256
-// bytes of a row; one thread per 8 consecutive k. Bound by the bf16 store:
-// 7168x5120, 73 MB: 23 us with one thread per word along a row, 16.6 us so.
+// groups, IT rounds of 8 rows), so that every 16 lanes write 256 bytes of a row;
+// one thread per 8 consecutive k. Bound by the bf16 store: 7168x5120, 73 MB: 25.8
+// us with one thread per word along a row, 23.3 with a workgroup per whole tile, 21.0 so.
 constexpr int kDeqGroups = 2;
+constexpr int kDeqRows = 256 / (16 * kDeqGroups);   // rows a workgroup does at once
+constexpr int kDeqIters = kTileN / kDeqRows;        // rounds over a tile's rows
 
+// IT of a tile's rounds per workgroup.
+template <int IT>
 __global__ __launch_bounds__(256) void k_dequant_rows(uint16_t* __restrict__ dst,
                                                       const uint32_t* __restrict__ qw,
                                                       const uint16_t* __restrict__ sc,
                                                       const uint16_t* __restrict__ zr, int row0,
                                                       int nrows, int K, int G) {
+  constexpr int kParts = kDeqIters / IT;
   const int per_tile = (G + kDeqGroups - 1) / kDeqGroups;
-  const int b = (row0 >> 6) + (int)blockIdx.x / per_tile;   // tile
-  const int g0 = ((int)blockIdx.x % per_tile) * kDeqGroups;
-  // thread: word wi of its group (of kDeqGroups), row `rs` of every 256 / (16
-  // kDeqGroups) rows
-  constexpr int kRows = 256 / (16 * kDeqGroups);
+  const int part = (int)blockIdx.x % kParts, item = (int)blockIdx.x / kParts;
+  const int b = (row0 >> 6) + item / per_tile;   // tile
+  const int g0 = (item % per_tile) * kDeqGroups;
+  // thread: word wi of its group (of kDeqGroups), row `rs` of every kDeqRows rows
   const int wi = threadIdx.x % (16 * kDeqGroups), rs = threadIdx.x / (16 * kDeqGroups);
   const int g = g0 + wi / 16, j = (wi >> 2) & 3, w = wi & 3;
   if (g >= G) return;
   const size_t blk = (size_t)b * G + g;
 #pragma unroll
-  for (int it = 0; it < kTileN / kRows; ++it) {
-    const int rr = rs + kRows * it, n = b * kTileN + rr;   // row of the tile, of the tensor
+  for (int it = 0; it < IT; ++it) {
+    const int rr = rs + kDeqRows * (part * IT + it), n = b * kTileN + rr;   // row of the tile, of the tensor
     if (n < row0 || n >= row0 + nrows) continue;
     const uint32_t word = qw[blk * kWordsPerBlock + j * 256 + tile_pos_of_row(rr) * 4 + w];
     const float s = bf16_bits_to_f32(sc[blk * kMetaU16 + rr]);
@@ -558,9 +562,16 @@ int qw4_dequant_rows(uint16_t* dst, const qw4_weights* w, int row0, int nrows, v
   if (((uintptr_t)dst & 15) != 0) return QW4_ERR_ALIGN;
   if (nrows == 0) return QW4_OK;
   const int tiles = ((row0 + nrows - 1) >> 6) - (row0 >> 6) + 1;
-  const unsigned nb = (unsigned)tiles * ((w->num_groups + kDeqGroups - 1) / kDeqGroups);
-  k_dequant_rows<<<nb, 256, 0, (hipStream_t)stream>>>(dst, w->qweight, w->scale, w->zeros, row0, nrows,
-                                                      w->in_f, w->num_groups);
+  const unsigned items = (unsigned)tiles * ((w->num_groups + kDeqGroups - 1) / kDeqGroups);
+  // One round of rows per workgroup where that is what fills the CUs, two beyond
+  // (64 / 512 / 5120 rows of K = 4096, us: eight rounds 3.8 / 4.9 / 15.4, one 2.3 / 3.5 /
+  // 15.7, two 2.4 / 3.4 / 13.3)
+  if (items <= 160)
+    k_dequant_rows<1><<<items * kDeqIters, 256, 0, (hipStream_t)stream>>>(
+        dst, w->qweight, w->scale, w->zeros, row0, nrows, w->in_f, w->num_groups);
+  else
+    k_dequant_rows<2><<<items * (kDeqIters / 2), 256, 0, (hipStream_t)stream>>>(
+        dst, w->qweight, w->scale, w->zeros, row0, nrows, w->in_f, w->num_groups);
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }

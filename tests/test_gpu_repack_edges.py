@@ -37,3 +37,24 @@ def test_repack_dequant_edges(orc, N, K, layout):
     m = orc.parity_metrics(host(y, np.uint16), orc.matmul_f64(x, q, zp, s, round_w=True))
     assert m["max_rel"] <= 1e-2 and m["mean_abs_vs_bf16_ref"] <= 1e-3, m
     hip.awq_free(w)
+
+
+# the two launch shapes of the row dequant: up to 160 (tile, two groups) items one
+# round of rows a workgroup, two beyond
+@pytest.mark.parametrize("N,K", [(640, 4096), (704, 4096), (768, 3712)])
+def test_dequant_launch_shapes(orc, N, K):
+    import torch
+    import w4a16_hip as hip
+
+    q, zp, s = orc.gen_weights(N, K, seed=N + K)
+    want = orc.dequant_bf16(q, zp, s)
+    w = repack_from_logical(hip, orc, q, zp, s, "ct")
+    for row0, n in ((0, N), (1, N - 2), (63, 66), (127, 1)):
+        print(f"dequant {N}x{K} rows {row0}+{n}", flush=True)
+        out = torch.full((n + 1, K), 0x5A5A, dtype=torch.int16, device="cuda")
+        hip.w4a16_dequant_rows(out[:n], w, row0, n)
+        torch.cuda.synchronize()
+        got = host(out, np.uint16)
+        assert np.array_equal(got[:n], want[row0:row0 + n])
+        assert (got[n] == 0x5A5A).all()
+    hip.awq_free(w)
