@@ -35,13 +35,20 @@ __device__ __forceinline__ uint32_t ct_to_slots(uint32_t s) {
   return ((ev | (ev >> 8)) & 0xFFFFu) | ((od | (od >> 8)) << 16);
 }
 
-// One wave per (tile, kRepackGroups groups), lane p at storage position p (row
+// One wave per (tile, two groups), lane p at storage position p (row
 // 4 (p % 16) + p / 16): whole 1 KiB of a block per store, and for source 0 the
 // 128 contiguous bytes of a row that one lane needs. The scale records and
 // zero points of the same groups go with them (lane r at row r), so a repack
 // is one launch. Bound by memory: 5120x5120 compressed-tensors, 27 MB
 // moved, 23 us in two launches with one thread per word, 10.2 us so.
-constexpr int kRepackGroups = 2;
+// Source 2 spreads the 8 k of a word over 8 source rows, 32 loads for a lane's 16
+// bytes: there a wave takes one chunk of one group (5120x512 / 5120x17408 7.6 / 39.4
+// us with two whole groups a wave, 6.2 / 24.2 so).
+template <int SRC>
+struct RepackItem {
+  static constexpr int kGroups = SRC == 2 ? 1 : 2;   // groups of a wave
+  static constexpr int kChunks = SRC == 2 ? 1 : 4;   // of the block's four 1 KiB chunks
+};
 
 template <int SRC>
 __global__ __launch_bounds__(256) void k_repack(uint32_t* __restrict__ dst,
@@ -52,18 +59,21 @@ __global__ __launch_bounds__(256) void k_repack(uint32_t* __restrict__ dst,
                                                 const uint32_t* __restrict__ szero, int n_src,
                                                 int K, int G, int tile0) {
   const int lane = threadIdx.x & 63;
-  const int per_tile = (G + kRepackGroups - 1) / kRepackGroups;
-  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int kGr = RepackItem<SRC>::kGroups, kCh = RepackItem<SRC>::kChunks;
+  const int per_tile = (G + kGr - 1) / kGr;
+  int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int j0 = item % (4 / kCh) * kCh;   // the item's first chunk
+  item /= 4 / kCh;
   if (item >= (n_src / kTileN) * per_tile) return;
-  const int bl = item / per_tile, g0 = (item % per_tile) * kRepackGroups;
+  const int bl = item / per_tile, g0 = (item % per_tile) * kGr;
   const int ns = bl * kTileN + tile_row_of_pos(lane);   // source row of position `lane`
-  u32x4 q[kRepackGroups][4];
+  u32x4 q[kGr][kCh];
 #pragma unroll
-  for (int i = 0; i < kRepackGroups; ++i) {
+  for (int i = 0; i < kGr; ++i) {
     const int g = min(g0 + i, G - 1);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = g * 16 + 4 * j;   // words r .. r + 3 of the row: k = 8 r .. 8 r + 31
+    for (int j = 0; j < kCh; ++j) {
+      const int r = g * 16 + 4 * (j0 + j);   // words r .. r + 3 of the row: k = 8 r .. 8 r + 31
       if (SRC == 0) {
         const uint32_t* s = src + (size_t)ns * (K / 8) + r;
 #pragma unroll
@@ -87,18 +97,19 @@ __global__ __launch_bounds__(256) void k_repack(uint32_t* __restrict__ dst,
     }
   }
 #pragma unroll
-  for (int i = 0; i < kRepackGroups; ++i) {
+  for (int i = 0; i < kGr; ++i) {
     const int g = g0 + i;
     if (g >= G) break;
     const size_t blk = (size_t)(tile0 + bl) * G + g;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kCh; ++j) {
       u32x4 o = q[i][j];
       if (SRC == 0)
 #pragma unroll
         for (int w = 0; w < 4; ++w) o[w] = ct_to_slots(o[w]);
-      *reinterpret_cast<u32x4*>(dst + blk * kWordsPerBlock + j * 256 + lane * 4) = o;
+      *reinterpret_cast<u32x4*>(dst + blk * kWordsPerBlock + (j0 + j) * 256 + lane * 4) = o;
     }
+    if (kCh < 4 && j0 != 0) continue;   // the record goes with the first chunk
     const int rn = bl * kTileN + lane;   // source row of the record's lane
     uint16_t sc;
     uint32_t z;
@@ -516,8 +527,8 @@ static int repack_into(qw4_weights* w, int row_offset, const uint32_t* q, const 
     return QW4_ERR_SHAPE;
   hipStream_t hs = (hipStream_t)stream;
   const int G = w->num_groups, tile0 = row_offset / kTileN;
-  const size_t items = (size_t)(out_f / kTileN) * ((G + kRepackGroups - 1) / kRepackGroups);
-  const unsigned nb = blocks_for(items, 4);
+  const size_t tiles = (size_t)(out_f / kTileN);
+  const unsigned nb = blocks_for(tiles * ((G + 1) / 2), 4);   // waves of RepackItem<0>, <1>
   switch (src) {
     case 0:
       k_repack<0><<<nb, 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
@@ -526,7 +537,7 @@ static int repack_into(qw4_weights* w, int row_offset, const uint32_t* q, const 
       k_repack<1><<<nb, 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
       break;
     case QW4_LAYOUT_AWQ_N:
-      k_repack<2><<<nb, 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
+      k_repack<2><<<blocks_for(tiles * G * 4, 4), 256, 0, hs>>>(w->qweight, w->scale, w->zeros, q, s, z, out_f, w->in_f, G, tile0);
       break;
     default:
       return QW4_ERR_LAYOUT;
