@@ -1,7 +1,8 @@
 """The decode kernel's launch shapes at the edges of their rules: the largest
 output that takes 16 waves (CUs / 4 tiles) and the next, the outputs on either
 side of one 64-row unit per workgroup, several units with a remainder, a K just
-below and at 32 groups, a K whose LDS leaves no room for 64-row units. Against
+below and at 32 groups, a K whose LDS leaves no room for 64-row units, more than
+eight 32- and 64-row units per workgroup (a second load of the residual). Against
 the oracle; the residual and swiglu epilogues bitwise against the plain
 projection followed by the separate step."""
 import numpy as np
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("N,G", [(4096, 31), (4096, 32), (4160, 40), (64, 40), (8192, 33), (8320, 33),
                                  (16384, 8), (16512, 8), (24704, 5), (9600, 25), (8320, 200),
-                                 (128, 64), (4096, 65)])
+                                 (128, 64), (4096, 65), (83200, 2), (163840, 2)])
 def test_dec_shapes(orc, N, G):
     import torch
 
