@@ -293,25 +293,27 @@ void launch(const SkinnyArgs& a, bool prepare, hipStream_t st) {
 }
 
 // Registers for 3, 5 or 8 groups a wave (K up to 3072, 5120, 8192): 110 to 210
-// of the 256, no spills.
-template <int OUT, int FMT, int S, int D>
+// of the 256, no spills. D3: items in flight where a wave has at most 3 groups.
+template <int OUT, int FMT, int S, int D, int D3 = D>
 void launch_ng(const SkinnyArgs& a, bool prepare, hipStream_t st) {
   const int ng = (a.G + kXrW - 1) / kXrW;
-  if (prepare || ng <= 3) launch<OUT, FMT, S, 3, D>(a, prepare, st);
+  if (prepare || ng <= 3) launch<OUT, FMT, S, 3, D3>(a, prepare, st);
   if (prepare || (ng > 3 && ng <= 5)) launch<OUT, FMT, S, 5, D>(a, prepare, st);
   if (prepare || ng > 5) launch<OUT, FMT, S, kXrMaxGroups, D>(a, prepare, st);
 }
 
 // Items in flight a wave: 4-bit 32-row units 3 (gate|up at M = 9: 2 19.9, 3
 // 19.3, 4 20.1 us; 6 was 7% slower), 16-row units 4; 8-bit 16-row units 2 (the
-// 248320-row head at M = 9: 2 214, 4 216, 6 217 us; 32-row units 222).
+// 248320-row head at M = 9: 2 214, 4 216, 6 217 us; 32-row units 222), but 4 for a
+// short K, whose units end sooner (151936x1024 / 151936x2560 / 32064x2560 at M = 9: 2
+// 34.9 / 71.8 / 18.9, 4 31.2 / 68.4 / 18.4, 6 32.5 / 70.8 / 19.4, k_rows 34.0 / 70.8 / 19.3).
 template <int OUT, int FMT>
 void launch_out(const SkinnyArgs& a, int S, bool prepare, hipStream_t st) {
   if constexpr (FMT == 4) {
     if (prepare || S == 1) launch_ng<OUT, FMT, 1, 4>(a, prepare, st);
     if (prepare || S == 2) launch_ng<OUT, FMT, 2, 3>(a, prepare, st);
   } else {
-    launch_ng<OUT, FMT, 1, 2>(a, prepare, st);
+    launch_ng<OUT, FMT, 1, 2, 4>(a, prepare, st);
   }
 }
 
@@ -352,9 +354,11 @@ bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, hipStream_t st) {
   a.U = a.tiles * 4 / S;
   // as few workgroups as give none of them another unit: each brings all rows of
   // x (34816x5120 at M = 9 / 16: 218 workgroups of 5 units 19.0 / 20.3 us, 256 of 4 or
-  // 5 20.5 / 22.1)
+  // 5 20.5 / 22.1); the 8-bit heads own tens of units each, and with a short K every
+  // workgroup streams for longer than it loads rows (151936x2560 at M = 9: 69.9 us
+  // with 250 workgroups, 68.4 with 256)
   const int n = out == OUT_SWIGLU ? a.U / 2 : a.U, most = (n + cus - 1) / cus;
-  a.P = (n + most - 1) / most;
+  a.P = fmt == 8 && a.G <= 3 * kXrW ? std::min(n, cus) : (n + most - 1) / most;
   dispatch(out, fmt, a, S, false, st);
   return true;
 }

@@ -82,7 +82,7 @@ def test_rows_xr_bitwise(hip, orc, scratch, N, G):
     hip.awq_free(w)
 
 
-@pytest.mark.parametrize("N,G", [(8256, 7), (8256, 40), (16448, 64), (192, 9)])
+@pytest.mark.parametrize("N,G", [(8256, 7), (8256, 40), (16448, 64), (192, 9), (20032, 20), (8256, 24), (8256, 25)])
 def test_rows_xr_w8_bitwise(hip, orc, scratch, N, G):
     K = 128 * G
     src = dev(orc.gen_x(N, K, seed=N + G))
