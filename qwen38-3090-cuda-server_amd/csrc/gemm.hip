@@ -87,6 +87,8 @@ struct G2Split {
   static constexpr int ACT = 8 * MB / NW;            // 1 KiB (4-row) activation loads per wave and group
   static constexpr int FIXP = (UNITS + 1) / 2;       // fixup blocks per wave region
   // groups buffered: as many 8 MB KiB activation buffers as LDS holds, 4 at most
+  // (MB = 5: three buffers spill 14 VGPRs, 60 bytes a lane, and are still faster
+  // than two without a spill: whole tiles 3%, split-K 1%, the others equal)
   static constexpr int DEPTH = MB <= 4 ? 4 : MB == 5 ? 3 : 2;
   // k-step schedule (measured on MI355X at the config-4 shapes): VALU slots
   // after each MFMA, LDS operand reads after each of the first MFMAs, and the
@@ -667,8 +669,11 @@ struct GemmPlan {
 
 // Time of one (tile, group) step by its m-blocks, relative to 8. Measured over
 // whole rounds of tiles (65536x5120, 256 and 1000 rows; us per 40 groups): 2 60,
-// 3 74, 4 91, 5 101, 6 110, 7 125, 8 145; 2 and 3 are charged a little more
-// for the memory latency that they expose when tiles are split.
+// 3 74, 4 91, 5 101, 6 110, 7 125, 8 145; 2, 3, 6 and 7 are charged 5 to 20% more,
+// for the memory latency that they expose when tiles are split. Over 12 projections
+// x 12 row counts from 48 to 1500, timed at every height and schedule, the plan's
+// pick is 1.3% (geometric mean) from the fastest; with the figures above as they
+// are 1.2%, but up to 5% slower than 256-row tiles.
 double step_cost(int mb) { return mb < 4 ? 0.38 + 0.06 * mb : 0.22 + 0.0975 * mb; }
 
 GemmPlan gemm_plan(int M, int N, long long G, int mb, int cus, bool ws_ok, int schedule) {
@@ -776,11 +781,17 @@ int qw4_gemm(uint16_t* C, const qw4_weights* w, const uint16_t* A, int M, qw4_wo
     // 66, o 5120x4096 36 / 36 / 40 -> 19 / 23 / 31), and few tiles, cut in fewer
     // slices (o at 256 rows 37 -> 28). By 3% at least, what the model resolves:
     // down at 2000 rows costs 100.9 in 224-row tiles against 101.3 and is 3% slower.
-    if (schedule == -1)
+    // Stream-K and hybrid of lower tiles by 7% against 256 rows: the cost of a
+    // workgroup's second segment does not shrink with the tile (9472x8448 at 500 / 1000
+    // rows, 128-row tiles costed at 0.93 / 0.95 of 256-row ones: 96.7 / 164 us against
+    // 94.0 / 155).
+    if (schedule == -1) {
+      const double cost8 = p.cost;
       for (int mb = 7; mb >= 2; --mb) {
         const GemmPlan q = gemm_plan(M, w->out_f, w->num_groups, mb, cus, ws_ok, schedule);
-        if (q.cost < 0.97 * p.cost) p = q;
+        if (q.cost < 0.97 * p.cost && !((q.pick == 1 || q.pick == 2) && q.cost >= 0.93 * cost8)) p = q;
       }
+    }
     const int nt = p.tiles_n * p.tiles_m, mb = p.mb;
     GemmArgs a{w->qweight, w->scale, w->zeros, A, C, nullptr, M, w->out_f, w->in_f,
                 w->num_groups, p.tiles_n, p.tiles_m, nt % 8 == 0, 32 * mb, nt, nt, 0};
