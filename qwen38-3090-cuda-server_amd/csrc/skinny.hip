@@ -1123,6 +1123,24 @@ int rows_occ(int S, bool xl) {
                   : rows_wgs_per_cu<OUT, FMT, 1, W>(xl);
 }
 
+// Outputs that M > 1 rows have (fp32 logits are M = 1 only, OUT_NORM's rows are
+// normalized in the staging).
+template <int OUT>
+constexpr bool rows_many() {
+  return OUT != OUT_NORM && OUT != OUT_F32;
+}
+
+// LDS of LDS-DMA items that bring their activation rows along: the slots and the
+// unit sums. Two items of 32-row units fit; three, or 64-row units, do not.
+template <int FMT>
+constexpr int rows_dma_need(int S, int D) {
+  return 8 * D * ((FMT == 8 ? 2 * S : S) * 1024 + 256 + 4096) + (FMT == 8 ? 1 : 2) * 8 * S * 64 * 16;
+}
+static_assert(rows_dma_need<4>(2, 2) <= kLdsBytes && rows_dma_need<8>(2, 2) <= kLdsBytes &&
+                  rows_dma_need<4>(2, 3) > kLdsBytes && rows_dma_need<8>(2, 3) > kLdsBytes &&
+                  rows_dma_need<4>(4, 2) > kLdsBytes && rows_dma_need<8>(4, 2) > kLdsBytes,
+              "the one form that launch_rows has");
+
 // k_rows policy (measured on MI355X over the model's projections, their 8-way
 // shards and the heads): S = 1 (16-row units) when the output has fewer
 // 64-row tiles than CUs / 4 (a 896-row shard: 4.7 vs 5.6 us), S = 2 when it
@@ -1190,13 +1208,14 @@ Launch launch_for(int out_f, int G, int M) {
       const long long pc2 = (long long)cus * (kLdsBytes / need);
       l.P = (int)std::max<long long>(1, std::min(OUT == OUT_SWIGLU ? u2 / 2 : u2, pc2));
     }
-  } else if (M > 1 && OUT != OUT_NORM && l.S != 1) {
+  } else if (M > 1 && rows_many<OUT>() && l.S != 1) {
     // All M rows staged in LDS once (padded rows, 32-row units, 2 items per
     // wave, one reduction buffer) when they fit and the workgroups own more
-    // than one unit on average: the per-item loads re-read x once per unit.
-    // Measured on MI355X, both forms in one process: gate|up at M = 9 (4.25
-    // units per workgroup) 22.3 against 24.1 us; with one unit per workgroup
-    // (qkv, o_proj) within +-5% either way, so those keep the per-item loads.
+    // than one unit on average: the per-item loads re-read x once per unit
+    // (what k_rows_xr takes does not come here). Measured on MI355X, both forms
+    // in one process, M = 4: 26624x9216 27.3 against 30.9 us, 35968x10240 37.2
+    // against 38.4, 49152x8448 38.4 against 40.4; with one unit per workgroup
+    // within +-5% either way, so those keep the per-item loads.
     const int xm_need = M * (G * kGroup * 2 + 16) +
                         8 * 2 * ((FMT == 8 ? 4 : 2) * 1024 + 256) +
                         8 * 2 * 64 * 16 + 512;
@@ -1211,11 +1230,12 @@ Launch launch_for(int out_f, int G, int M) {
       l.P = (int)std::max<long long>(1, std::min(OUT == OUT_SWIGLU ? u2 / 2 : u2, (long long)cus));
       return l;
     }
-    if constexpr (FMT == 4 && (OUT == OUT_BF16 || OUT == OUT_F32 || OUT == OUT_RES)) {
+    if constexpr (FMT == 4 && (OUT == OUT_BF16 || OUT == OUT_RES)) {
       // Otherwise, several units per workgroup: group-major items, each
       // activation group fetched once per workgroup (k_rows_gm). Measured on
-      // MI355X, gate|up at M = 16: 24.2 against 28.1 us for the per-item
-      // loads; at M = 9 the staged rows above stay faster (23.7 against 24.1).
+      // MI355X against the per-item loads, M = 9 / 16: 24576x8448 24.1 / 24.1 against
+      // 23.6 / 27.6 us, 26624x9216 29.8 / 30.5 against 31.1 / 36.7, 35968x10240 38.8 /
+      // 40.3 against 42.5 / 51.8, 49152x8448 40.0 / 40.9 against 44.5 / 51.6.
       const long long u2 = (long long)tiles * 2;
       const long long pg = std::min<long long>(u2, cus);
       if (mode != 1 && mode != 2 && mode != 4 && mode != 5 && u2 / pg >= kGmMinU &&
@@ -1230,19 +1250,14 @@ Launch launch_for(int out_f, int G, int M) {
       }
     }
     int S = l.S;
-    const int dd = (mode == 1 && tD >= 2 && tD <= 4 && !(OUT == OUT_ARGMAX && S == 4)) ? tD : 2;
-    // weights, metadata and the item's 16 activation rows (rows_slot_units)
-    auto need_for = [&](int s_) {
-      const int slot = (FMT == 8 ? 2 * s_ : s_) * 1024 + 256 + 4096;
-      return 8 * dd * slot + (FMT == 8 ? 1 : 2) * 8 * s_ * 64 * 16;
-    };
+    const int dd = (mode == 1 && tD >= 2 && tD <= 4) ? tD : 2;
     // 64-row units whose slots do not fit: 32-row units with the activations
     // in the slots (measured on MI355X: gate|up at M = 16, 28.1 us against 29.6
     // for 64-row units with the activations loaded into registers)
     // (4-bit only: the 8-bit head at M = 9 keeps its 64-row register form,
     // 352 against 368 us for 32-row units with the activations in the slots)
-    if (FMT == 4 && S == 4 && need_for(4) > kLdsBytes && !(mode == 1 && tS == 4)) S = 2;
-    const int need = need_for(S);
+    if (FMT == 4 && S == 4 && !(mode == 1 && tS == 4)) S = 2;
+    const int need = rows_dma_need<FMT>(S, dd);
     if (need <= kLdsBytes) {
       l.S = S;
       l.DMA = dd;
@@ -1426,22 +1441,15 @@ void prepare_gm() {
     allow_lds<kern>(kLdsBytes - (int)at.sharedSizeBytes);
 }
 
-// Every LDS-DMA kernel the launch code can pick (launch_rows_dma).
+// Every LDS-DMA kernel the launch code can pick (launch_rows).
 template <int OUT, int FMT>
 void prepare_dma_out() {
   prepare_dma_one<OUT, FMT, 2, true, 2>();
   prepare_dma_one<OUT, FMT, 2, true, 3>();
   prepare_dma_one<OUT, FMT, 2, true, 4>();
-  if constexpr (OUT != OUT_NORM) {
+  if constexpr (rows_many<OUT>()) {
     prepare_dma_one<OUT, FMT, 2, true, 2, true>();
     prepare_dma_one<OUT, FMT, 2, false, 2>();
-    prepare_dma_one<OUT, FMT, 2, false, 3>();
-    prepare_dma_one<OUT, FMT, 2, false, 4>();
-    prepare_dma_one<OUT, FMT, 4, false, 2>();
-    if constexpr (OUT != OUT_ARGMAX) {
-      prepare_dma_one<OUT, FMT, 4, false, 3>();
-      prepare_dma_one<OUT, FMT, 4, false, 4>();
-    }
   }
 }
 
@@ -1456,7 +1464,6 @@ void prepare_dma_lds() {
     prepare_dec<OUT_NORM>();
     rows_xr_prepare();
     prepare_gm<OUT_BF16>();
-    prepare_gm<OUT_F32>();
     prepare_gm<OUT_RES>();
     prepare_dma_out<OUT_BF16, 4>();
     prepare_dma_out<OUT_F32, 4>();
@@ -1469,22 +1476,6 @@ void prepare_dma_lds() {
   });
 }
 
-// LDS-DMA items: units of S row quads, 8 waves, D items per wave; staged
-// activations (M = 1, S = 2) or activations loaded with each item (M > 1)
-template <int OUT, int FMT, int S, bool XL>
-void launch_rows_dma(const SkinnyArgs& a, int D, hipStream_t st) {
-  if constexpr (OUT == OUT_ARGMAX && S == 4) {   // deeper would spill (launch_for caps D)
-    launch_rows_dma_d<OUT, FMT, S, 8, 2, XL>(a, st);
-  } else {
-    if (D == 2)
-      launch_rows_dma_d<OUT, FMT, S, 8, 2, XL>(a, st);
-    else if (D == 3)
-      launch_rows_dma_d<OUT, FMT, S, 8, 3, XL>(a, st);
-    else
-      launch_rows_dma_d<OUT, FMT, S, 8, 4, XL>(a, st);
-  }
-}
-
 template <int OUT>
 void launch_rows_gm(const SkinnyArgs& a, hipStream_t st) {
   const int lds = 8 * gm_wave_units() * 16;
@@ -1495,27 +1486,31 @@ void launch_rows_gm(const SkinnyArgs& a, hipStream_t st) {
 
 template <int OUT, int FMT>
 void launch_rows(const SkinnyArgs& a, const Launch& l, hipStream_t st) {
-  if constexpr (FMT == 4 && (OUT == OUT_BF16 || OUT == OUT_F32 || OUT == OUT_RES)) {
+  if constexpr (FMT == 4 && (OUT == OUT_BF16 || OUT == OUT_RES)) {
     if (l.GM) {
       launch_rows_gm<OUT>(a, st);
       return;
     }
   }
   if (l.DMA) {
-    if constexpr (OUT != OUT_NORM) {
-      if (l.XM) {   // M > 1 rows staged: 2 items per wave (launch_for)
+    // LDS-DMA items, 32-row units, 8 waves: M = 1 staged, l.DMA items per wave;
+    // M > 1 staged (XM) or brought by each item, 2 items per wave
+    if constexpr (rows_many<OUT>()) {
+      if (l.XM) {
         launch_rows_dma_d<OUT, FMT, 2, 8, 2, true, true>(a, st);
         return;
       }
+      if (!l.XL) {
+        launch_rows_dma_d<OUT, FMT, 2, 8, 2, false>(a, st);
+        return;
+      }
     }
-    if (l.XL)
-      launch_rows_dma<OUT, FMT, 2, true>(a, l.DMA, st);
-    else if constexpr (OUT != OUT_NORM) {
-      if (l.S == 4)
-        launch_rows_dma<OUT, FMT, 4, false>(a, l.DMA, st);
-      else
-        launch_rows_dma<OUT, FMT, 2, false>(a, l.DMA, st);
-    }
+    if (l.DMA == 2)
+      launch_rows_dma_d<OUT, FMT, 2, 8, 2, true>(a, st);
+    else if (l.DMA == 3)
+      launch_rows_dma_d<OUT, FMT, 2, 8, 3, true>(a, st);
+    else
+      launch_rows_dma_d<OUT, FMT, 2, 8, 4, true>(a, st);
     return;
   }
   if (OUT == OUT_ARGMAX || l.W == 8)
