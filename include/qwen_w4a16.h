@@ -136,15 +136,17 @@ int qw4_choose_splits(int out_f, int num_groups);
  * registers for every M, S (1, 2, 4 row quads per unit) and W (8, 16 waves)
  * forcing its shape; 3 the decode kernel with unit size S, W waves and D items
  * per wave (0 = the policy's value); 4 the policy with the M > 1 activations
- * never staged in LDS and never shared by a workgroup's units (loaded with
- * each item); 5 the policy without the group-major M > 1 kernel. P > 0 forces
- * the decode kernel's workgroup count. */
+ * loaded with each item (never held in registers, staged in LDS or shared by a
+ * workgroup's units); 5 the policy without the M > 1 kernels that hold the
+ * activations in registers (k_rows_xr) or go group by group (k_rows_gm). Modes 1
+ * to 5 also keep qw4_linear's passes at 16 rows. P > 0 forces the decode kernel's
+ * workgroup count. */
 int qw4_tune_decode(int mode, int S, int W, int D, int P);
 /* qw4_tune_gemm: the prefill schedule, -1 the cost model (default), 0 one
  * workgroup per tile, 1 stream-K, 2 hybrid, 3 split-K (every tile cut into the
  * same k-slices; at most CUs / 2 tiles) (split schedules need a workspace);
  * variant 0 the default kernel (4 waves, each on a whole 64-row weight tile
- * against all activation rows of the workgroup's tile, 32 to 256), 1 8 waves
+ * against all activation rows of the workgroup's tile, 64 to 256), 1 8 waves
  * on 32-row tile halves, 2 8 waves on whole tiles against half the rows (both
  * computing 256 rows whatever the tile's); under every schedule the variants'
  * results are bitwise equal. */

@@ -405,8 +405,9 @@ __global__ __launch_bounds__(64 * W) void k_rows(SkinnyArgs a) {
 }
 
 // ------------------------------------- verify, several units per workgroup
-// k_rows_gm: M > 1, 4-bit weights, 32-row units, 8 waves, for shapes where
-// every workgroup owns n units, kGmMinU <= n <= kGmMaxU (gate|up: 4 or 5).
+// k_rows_gm: M > 1, 4-bit weights, 32-row units, 8 waves, for shapes that k_rows_xr
+// cannot hold (K > 8192) and where every workgroup owns n units, kGmMinU <= n <=
+// kGmMaxU (24576 to 49152 rows on 256 CUs).
 // k_rows loads an item's group of the 16 activation rows with every item, so
 // a workgroup fetches each activation group n times; here the items run
 // group-major -- wave w takes groups g = w + W gi and, for each, first loads
@@ -1038,7 +1039,8 @@ struct DecTune {
   // 0 policy; 1 k_rows for M = 1 too (S forces the unit size, D the LDS-DMA
   // depth 2..4); 2 k_rows with register items (S / W force unit size, waves);
   // 3 k_dec of the given S / W / D (OUT_BF16); 4 the policy, but M > 1 rows
-  // never staged in LDS (activations loaded with each item)
+  // loaded with each item (k_rows; no k_rows_xr, k_rows_gm, staged rows); 5 the
+  // policy without k_rows_xr and k_rows_gm
   std::atomic<int> mode{0};
   std::atomic<int> S{0}, W{0}, D{0}, P{0};
 };
@@ -1840,11 +1842,14 @@ int qw4_gemv_residual(uint16_t* h, const qw4_weights* w, const uint16_t* x, int 
 int qw4_gemv_swiglu(uint16_t* y, const qw4_weights* w, const uint16_t* x, int M, uint16_t* tmp,
                     qw4_scratch* s, void* stream) {
   // Fused for M <= 2, and where the pairs fill one round of workgroups (more
-  // than CUs / 2 tiles, at most CUs: 8704x5120 at M = 9 10.0 us against 12.9, at
-  // 16384x5120 11.7 against 14.2). Elsewhere the pairing of gate and up rows in
-  // one workgroup is no faster than the projection plus a separate swiglu
-  // (17408x5120 16.6 against 16.7, 4352x5120 10.8 against 9.0), which runs through
-  // tmp when one is given.
+  // than CUs / 2 tiles, at most CUs), in k_rows_xr (us at M = 3 / 9 / 16 against the
+  // projection and a separate swiglu: 16384x1024 5.6 / 5.6 / 5.7, 7.4 / 7.6 / 7.8;
+  // 8704x5120 9.8 / 10.0 / 10.3, 11.8 / 11.9 / 12.4; 16384x7168 14.1 / 14.2 / 14.8, 15.2 /
+  // 16.0 / 17.0) and, beyond its K, in k_rows (8448x8448 15.0 / 15.1 / 17.7, 16.1 /
+  // 17.9 / 19.7; 16384x12288 21.8 / 23.4 / 26.3, 23.7 / 24.9 / 28.3; 8704x17408 27.4 /
+  // 27.5 / 32.8, 26.6 / 29.9 / 35.6). Elsewhere the pairing of gate and up rows in one
+  // workgroup is no faster (17408x5120 16.6 against 16.7 at M = 9, 4352x5120 10.8
+  // against 9.0), and the projection goes through tmp when one is given.
   const int tiles = w ? w->out_f / kTileN : 0, cus = device_cus();
   if (M <= 2 || !tmp || (2 * tiles > cus && tiles <= cus))
     return run_skinny<OUT_SWIGLU>(y, w, x, M, s, stream);

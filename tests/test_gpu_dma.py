@@ -300,13 +300,14 @@ def test_dma_w8_verify(hip, scratch, M):
 
 # ------------------------------------------- M > 1 with the rows staged in LDS
 def _staged_vs_per_item(hip, run):
-    """run() with the policy (the activation rows staged in LDS where they fit
-    and the workgroups own several units; else, with 3 to 6 units per
-    workgroup, the group-major kernel k_rows_gm), with per-item activation
-    loads (qw4_tune_decode mode 4), with register items (mode 2) and with the
-    group-major kernel off (mode 5): every result equal. The per-row sums run
-    over the same groups in the same wave order in every form, so any
-    difference is a staging, padding, slot-reuse or wait error."""
+    """run() with the policy (K up to 8192: k_rows_xr; beyond, the activation
+    rows staged in LDS where they fit and the workgroups own several units;
+    else, with 3 to 6 units per workgroup, the group-major kernel k_rows_gm),
+    with per-item activation loads (qw4_tune_decode mode 4), with register
+    items (mode 2) and without k_rows_xr and k_rows_gm (mode 5: staged rows
+    where they fit): every result equal. The per-row sums run over the same
+    groups in the same wave order in every form, so any difference is a
+    staging, padding, slot-reuse or wait error."""
     try:
         hip.tune_decode(0)
         want = run()
@@ -319,11 +320,11 @@ def _staged_vs_per_item(hip, run):
 
 
 # gate|up (544 tiles), a head-like 16384-row output, a short-K one; the 5120-row
-# output has fewer tiles than half the CUs and keeps the per-item loads. Where
-# the rows do not fit the staging (M = 12 / 16 on gate|up, the 3- and
-# 6-units-per-workgroup shapes) the group-major kernel runs.
+# output has fewer tiles than half the CUs and keeps the per-item loads. K = 8320
+# is beyond k_rows_xr: staged rows at M = 2, and at M = 9 .. 16, where they do not
+# fit, the group-major kernel with 3 or 4 and with 6 units per workgroup.
 STAGED = [(34816, 5120), (16384, 1024), (20480, 384), (5120, 4096), (24576, 5120),
-          (49152, 5120)]
+          (49152, 5120), (26624, 8320), (49152, 8320)]
 
 
 @pytest.mark.parametrize("M", [2, 9, 12, 16])
