@@ -1,5 +1,6 @@
 """Non-finite activations through the decode (M = 1, k_dec) and verify (M = 9,
-k_rows) kernels, through the C-ABI.
+k_rows; k_rows_xr where it runs, with one and two row blocks and its fused
+epilogues) kernels, through the C-ABI.
 
 The reference's fp32 GEMV adds per group p = sum_k (128 + q) x then subtracts
 (128 + zp) * sum_k x (src/kernels/gemv_w4a16.cu:136-147): an Inf or NaN
@@ -101,4 +102,65 @@ def test_subnormal_group_is_bounded(hip, orc, scratch):
     ref = orc.matmul_f64(x, q, zp, s)
     assert np.isfinite(got).all()
     assert np.max(np.abs(got - ref)) < 1e-30
+    hip.awq_free(w)
+
+
+@pytest.mark.parametrize("N,K,M", [(8320, 5120, 16), (8320, 8192, 9), (192, 1152, 12), (8320, 5120, 30),
+                                   (192, 1152, 32)])
+@pytest.mark.parametrize("bad", [BF16_INF, BF16_NINF, BF16_NAN])
+def test_nonfinite_rows_in_registers(hip, orc, scratch, N, K, M, bad):
+    """k_rows_xr: 8320 rows own several units a workgroup, 192 are few 16-row
+    units; more than 16 rows are qw4_linear's pass of two row blocks."""
+    import torch
+
+    q, zp, s = orc.gen_weights(N, K, seed=11)
+    w = repack_from_logical(hip, orc, q, zp, s, "awq_k")
+    x = orc.gen_x(M, K, seed=12).copy()
+    rows = [M // 2, M - 1]
+    xb = x.copy()
+    xb[rows[0], K - 1] = bad
+    xb[rows[1], 130] = bad
+    others = [m for m in range(M) if m not in rows]
+
+    def plain(v):
+        y = empty((M, N), np.uint16)
+        hip.linear_w4a16(y, w, dev(v), M, scratch)
+        torch.cuda.synchronize()
+        return host(y, np.uint16)
+
+    def swiglu(v):
+        y = empty((M, N // 2), np.uint16)
+        hip.gemv_swiglu_w4a16(y, w, dev(v), M, scratch)
+        torch.cuda.synchronize()
+        return host(y, np.uint16)
+
+    def argmax(v):
+        y = empty((M,), np.int32)
+        hip.gemv_argmax_w4a16(y, w, dev(v), M, scratch)
+        torch.cuda.synchronize()
+        return host(y, np.int32)
+
+    print(f"non-finite rows M={M} {N}x{K} bad={bad}", flush=True)
+    assert hip.linear_max_t(w) >= M
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = orc.matmul_f64(xb, q, zp, s)
+    got = plain(xb)
+    assert np.isnan(_bf16_to_f64(got[rows])).all()
+    assert np.array_equal(got[others], plain(x)[others])
+    m = orc.parity_metrics(got[others], ref[others])
+    assert m["max_rel"] <= 1e-2 and m["mean_abs_vs_bf16_ref"] <= 1e-3, m
+    if M <= 16:
+        runs = (argmax, swiglu) if N % 128 == 0 else (argmax,)
+        for run in runs:
+            got, clean = run(xb), run(x)
+            assert np.array_equal(got[others], clean[others])
+            try:
+                hip.tune_decode(2)   # register items of k_rows: the same sums
+                assert np.array_equal(got[others], run(xb)[others])
+                if run is argmax:
+                    assert np.array_equal(got, run(xb))
+            finally:
+                hip.tune_decode(0)
+        if N % 128 == 0:
+            assert np.isnan(_bf16_to_f64(swiglu(xb)[rows])).all()
     hip.awq_free(w)
