@@ -1316,7 +1316,10 @@ constexpr int kDecCount = (int)(sizeof(kDecAll) / sizeof(kDecAll[0]));
 //  * else 8, of 2 items for short outputs or K (qkv: 5.7 against 6.0; o_proj 4.9
 //    against 5.0), of 3 otherwise (gate|up).
 // Unit size: 32 rows, but 64 where no workgroup gets more rows for it -- half as
-// many items (8704x5120 7.5 -> 6.7 us, 9600x3200 6.3 -> 5.7). OUT_SWIGLU, whose
+// many items (8704x5120 7.5 -> 6.7 us, 9600x3200 6.3 -> 5.7); not for single units of a
+// K that gives half the waves no item (8320x640 4.08 us in 32-row units, 4.16 in 64,
+// 14720x640 4.42 and 4.49, with rmsnorm 5.34 and 5.77), with rmsnorm and many
+// workgroups not below 20 groups (14720x1280 5.77, 6.02; at 20 they meet). OUT_SWIGLU, whose
 // workgroups own whole (gate, up) pairs: 64 by the same rule (dec_swiglu_rows;
 // 17408x5120 12.7 -> 10.9 us), and 16 where that halves the rows of a single round
 // (4352x5120 7.3 -> 6.5; over several rounds it does not pay: 34816x5120 18.9
@@ -1337,6 +1340,7 @@ bool dec_config(int out_f, int G, int OUTmode, DecCfg& c) {
                                 : kDecAll[0];
   // 64-row units hold more in flight: only where a long K leaves the LDS
   const bool fits4 = dec_lds_units(K, G, OUTmode == OUT_NORM, 4, 8, 2) * 16 + dec_static_lds(4, 8) <= kLdsBytes;
+  const bool short_k = tiles <= cus && (G < 8 || (OUTmode == OUT_NORM && G < 20 && 4 * tiles > 3 * cus));
   if (v.W == 8) {
     if (OUTmode == OUT_SWIGLU) {
       const int r1 = dec_swiglu_rows(tiles, 1, cus), r2 = dec_swiglu_rows(tiles, 2, cus),
@@ -1345,7 +1349,7 @@ bool dec_config(int out_f, int G, int OUTmode, DecCfg& c) {
         v = kDecAll[4];
       else if (r1 < r2 && 2 * tiles <= cus)
         v = kDecAll[5];
-    } else if ((tiles + cus - 1) / cus * 64 <= (2 * tiles + cus - 1) / cus * 32 && fits4) {
+    } else if ((tiles + cus - 1) / cus * 64 <= (2 * tiles + cus - 1) / cus * 32 && fits4 && !short_k) {
       v = kDecAll[4];
     }
   }

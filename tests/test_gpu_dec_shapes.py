@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("N,G", [(4096, 31), (4096, 32), (4160, 40), (64, 40), (8192, 33), (8320, 33),
                                  (16384, 8), (16512, 8), (24704, 5), (9600, 25), (8320, 200),
-                                 (128, 64), (4096, 65), (83200, 2), (163840, 2)])
+                                 (128, 64), (4096, 65), (83200, 2), (163840, 2), (14720, 7), (16384, 5)])
 def test_dec_shapes(orc, N, G):
     import torch
 
