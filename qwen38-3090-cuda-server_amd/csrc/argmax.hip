@@ -65,11 +65,11 @@ __global__ __launch_bounds__(T) void k_argmax_rows(int32_t* out, const uint16_t*
 #pragma unroll
     for (int j = 0; j < kRowChunks; ++j) {
       const int kj = k + j * T;
-      if (j * T < left) d[j] = body[kj < chunks ? kj : k];   // past the end: chunk k again, never greater
+      if (T == 1024 || j * T < left) d[j] = body[kj < chunks ? kj : k];   // past the end: chunk k again, never greater
     }
 #pragma unroll
     for (int j = 0; j < kRowChunks; ++j) {
-      if (j * T >= left) break;   // uniform: a short row has fewer rounds of loads
+      if (T < 1024 && j * T >= left) break;   // uniform: a short row has fewer rounds of loads
       float m = -FLT_MAX;   // fmaxf passes over NaN
 #pragma unroll
       for (int e = 0; e < 4; ++e)
