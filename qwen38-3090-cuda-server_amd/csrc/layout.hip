@@ -3,6 +3,8 @@
 // bf16 dequant of repacked rows, status strings and the synthetic generator.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(256) void k_repack(uint32_t* __restrict__ dst,
 // dst [nrows][K] = RNE(float(q - z) * s). One workgroup per (tile, kDeqGroups
 // groups, IT rounds of 8 rows), so that every 16 lanes write 256 bytes of a row;
 // one thread per 8 consecutive k. Bound by the bf16 store: 7168x5120, 73 MB: 25.8
-// us with one thread per word along a row, 23.3 with a workgroup per whole tile, 21.0 so.
+// us with one thread per word along a row, 23.3 with a workgroup per whole tile, 20.3 so.
 constexpr int kDeqGroups = 2;
 constexpr int kDeqRows = 256 / (16 * kDeqGroups);   // rows a workgroup does at once
 constexpr int kDeqIters = kTileN / kDeqRows;        // rounds over a tile's rows
@@ -574,15 +576,21 @@ int qw4_dequant_rows(uint16_t* dst, const qw4_weights* w, int row0, int nrows, v
   if (nrows == 0) return QW4_OK;
   const int tiles = ((row0 + nrows - 1) >> 6) - (row0 >> 6) + 1;
   const unsigned items = (unsigned)tiles * ((w->num_groups + kDeqGroups - 1) / kDeqGroups);
-  // One round of rows per workgroup where that is what fills the CUs, two beyond
-  // (64 / 512 / 5120 rows of K = 4096, us: eight rounds 3.8 / 4.9 / 15.4, one 2.3 / 3.5 /
-  // 15.7, two 2.4 / 3.4 / 13.3)
+  // As many rounds of rows per workgroup as leave the CUs enough of them (us with
+  // one / two / four / eight: 64 rows of K = 4096 2.8 / 2.9 / 3.3 / 4.2, 512 rows of K =
+  // 5120 3.9 / 3.7 / 4.0 / 4.8, 2048 8.5 / 7.7 / 6.9 / 7.8, 7168 25.5 / 21.7 / 20.3 / 23.5;
+  // 7168 just repacked, three repacks included, 42.9 / 38.6 / 35.9 / 37.2)
+  const auto launch = [&](auto it) {
+    constexpr int kIt = decltype(it)::value;
+    k_dequant_rows<kIt><<<items * (kDeqIters / kIt), 256, 0, (hipStream_t)stream>>>(
+        dst, w->qweight, w->scale, w->zeros, row0, nrows, w->in_f, w->num_groups);
+  };
   if (items <= 160)
-    k_dequant_rows<1><<<items * kDeqIters, 256, 0, (hipStream_t)stream>>>(
-        dst, w->qweight, w->scale, w->zeros, row0, nrows, w->in_f, w->num_groups);
+    launch(std::integral_constant<int, 1>{});
+  else if (items <= 512)
+    launch(std::integral_constant<int, 2>{});
   else
-    k_dequant_rows<2><<<items * (kDeqIters / 2), 256, 0, (hipStream_t)stream>>>(
-        dst, w->qweight, w->scale, w->zeros, row0, nrows, w->in_f, w->num_groups);
+    launch(std::integral_constant<int, 4>{});
   QW4_LAUNCH_CHECK();
   return QW4_OK;
 }

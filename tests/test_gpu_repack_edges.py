@@ -39,9 +39,10 @@ def test_repack_dequant_edges(orc, N, K, layout):
     hip.awq_free(w)
 
 
-# the two launch shapes of the row dequant: up to 160 (tile, two groups) items one
-# round of rows a workgroup, two beyond
-@pytest.mark.parametrize("N,K", [(640, 4096), (704, 4096), (768, 3712)])
+# the launch shapes of the row dequant: up to 160 (tile, two groups) items one round
+# of rows a workgroup, up to 512 two, four beyond
+@pytest.mark.parametrize("N,K", [(640, 4096), (704, 4096), (768, 3712), (2048, 4096), (2112, 4096),
+                                 (2240, 3968)])
 def test_dequant_launch_shapes(orc, N, K):
     import torch
     import w4a16_hip as hip
