@@ -3,7 +3,7 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--layers 64] [--no-cpu]
                     [--only-decode | --only-verify | --only-prefill]
 
-Headline (BASELINE.json configs[1]): the decode GEMV sweep of a full layer --
+Headline: the decode GEMV sweep of a full layer --
 qkv (5120->7168), o (4096->5120), gate|up (5120->34816), down (17408->5120) --
 over 64 layers of distinct synthetic weights (10.07 GiB of algorithmic bytes,
 far beyond the 256 MB MALL). One step = one decoded token's body: all 256 GEMV

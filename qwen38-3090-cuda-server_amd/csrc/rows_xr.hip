@@ -353,8 +353,9 @@ bool rows_xr_launch(int out, int fmt, SkinnyArgs& a, int cus, hipStream_t st) {
   const int S = fmt == 8 || small ? 1 : 2;
   a.U = a.tiles * 4 / S;
   // as few workgroups as give none of them another unit: each brings all rows of
-  // x (34816x5120 at M = 9 / 16: 218 workgroups of 5 units 19.0 / 20.3 us, 256 of 4 or
-  // 5 20.5 / 22.1); the 8-bit heads own tens of units each, and with a short K every
+  // x (M = 2 / 9 / 16, against a workgroup per CU: 34816x5120 18.8 / 20.2 / 20.6 us, 19.2 /
+  // 20.0 / 20.7; 28672x4096 13.7 / 14.3 / 14.9, 13.9 / 14.7 / 15.4; 34816x8192 28.7 / 29.9 /
+  // 31.3, 29.2 / 31.7 / 31.7; 9472x5120 9.7 / 10.0 / 10.4, 9.3 / 9.9 / 10.6); the 8-bit heads own tens of units each, and with a short K every
   // workgroup streams for longer than it loads rows (151936x2560 at M = 9: 69.9 us
   // with 250 workgroups, 68.4 with 256)
   const int n = out == OUT_SWIGLU ? a.U / 2 : a.U, most = (n + cus - 1) / cus;

@@ -266,7 +266,7 @@ def awq_repack(packed, scale, zp, out_f: int, in_f: int, group_size: int = 128,
 
 def awq_repack_awq_into(w: W4A16Weights, row_offset: int, qweight, scales, zeros, out_f: int,
                         layout: int = LAYOUT_AWQ_K, stream=None) -> None:
-    """AWQ-order sources (BASELINE layout along K, or AutoAWQ along N)."""
+    """AWQ-order sources (packed along K, or along N as AutoAWQ does)."""
     G = w.in_f // 128
     _need(qweight, out_f * w.in_f // 2, "awq_repack_awq_into qweight")
     _need(scales, out_f * G * 2, "awq_repack_awq_into scales")
