@@ -47,10 +47,12 @@ def test_argmax_rows(orc, n, kind):
         assert np.array_equal(got, orc.argmax_rows_bf16(v))
 
 
-# the edges of the workgroup sizes: 64 threads up to 2048 values, 1024 for rows of
-# more than 24576 values in calls of at most 512 rows, 256 for the others
+# the edges of the workgroup sizes: 64 threads up to 2048 values (value by value up to
+# 128), 1024 for rows of more than 24576 values in calls of at most 512 rows, 256 for the
+# others
 @pytest.mark.parametrize("n,rows", [(2047, 300), (2048, 3), (2049, 300), (24576, 5), (24577, 5),
-                                    (24583, 512), (24583, 513), (3, 70000)])
+                                    (24583, 512), (24583, 513), (3, 70000), (63, 7),
+                                    (65, 7), (128, 40), (129, 40)])
 def test_argmax_rows_workgroups(orc, n, rows):
     import torch
     import w4a16_hip as hip
